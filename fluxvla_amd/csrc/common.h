@@ -223,6 +223,26 @@ __device__ __forceinline__ int xcd_remap(int bid, int nblk) {
   return x * per + (x < rem ? x : rem) + local;
 }
 
+// Tile `bid` of an m_tiles x n_tiles grid, in blocks of tile rows (at most
+// `most` of them, as even as they go): the blocks one after another, inside a
+// block m fastest.  The tiles that run together on an XCD (consecutive ids)
+// then cover about as many rows as columns, so that few panels of A and B
+// pass through its L2; down one whole column of tiles instead, every XCD
+// streams all of A.
+__device__ __forceinline__ void tile_order(int bid, int m_tiles, int n_tiles, int most, int& m,
+                                           int& n) {
+  if (m_tiles <= most) {  // one block, without its divisions
+    n = bid / m_tiles;
+    m = bid - n * m_tiles;
+    return;
+  }
+  const int ng = (m_tiles + most - 1) / most, gm = (m_tiles + ng - 1) / ng;
+  const int g = bid / (gm * n_tiles), r = bid - g * gm * n_tiles;
+  const int rows = m_tiles - g * gm < gm ? m_tiles - g * gm : gm;
+  n = r / rows;
+  m = g * gm + (r - n * rows);
+}
+
 typedef __attribute__((address_space(3))) char lds_char_t;
 
 __device__ __forceinline__ uint32_t lds_addr(const void* p) {

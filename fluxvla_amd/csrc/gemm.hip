@@ -22,9 +22,10 @@
 //  * gemm_partial_reduce_kernel: the split-K sum (in split order,
 //    deterministic) and epilogue behind the tile and wide kernels.
 //
-// Tiles are ordered m-fastest within a weight panel and block ids remapped
-// (xcd_remap) so that one XCD owns consecutive tiles: the m-tiles of a
-// panel run on one XCD and reuse the panel from its L2.
+// Tiles are ordered m-fastest within blocks of about 1024 rows (tile_order)
+// and block ids remapped (xcd_remap) so that one XCD owns consecutive tiles:
+// the tiles of a block run on one XCD and reuse its rows of A and its weight
+// panels from the L2.
 //
 // Per-row RMSNorm ("rownorm") is fused: the kernel that streams A also
 // accumulates sum(A[m][:]^2) (or takes the sums handed over by the GEMM that
@@ -44,6 +45,15 @@ typedef fvx_gemm_desc GemmArgs;
 // arrival counters of the split-K skinny kernel; fp32 partials follow.
 constexpr int kCounterBytes = 4096;
 constexpr int kMaxSkinnyTiles = kCounterBytes / 4;
+
+// Tile rows per block of the tile order (tile_order): about 1024 rows.  One
+// block of all rows against this, us (MI355X, weights from HBM): prefix down
+// 6528 x 2048 x 16384 538 -> 428 (all 26 tile rows on every XCD streamed A
+// eight times), gate/up 6528 x 2 x 16384 x 2048 775 -> 750, Q|K|V 107 -> 98;
+// SigLIP fc1 6144 x 4304 x 1152 97 -> 89, Q|K|V 81 -> 75, fc2 120 -> 114; fp8
+// gate/up at 22144 rows 2970 -> 2850.  Blocks of 2048 rows: gate/up 785.
+constexpr int kTileRowBlock = 16;  // tiles of 64 rows
+constexpr int kWideRowBlock = 4;   // tiles of 256 rows
 
 
 // Row indices and the epilogue's periods (row_group, gate_group,
@@ -752,7 +762,8 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void gemm_tile_kernel(
   const int nblk = m_tiles * n_tiles;
   const int lid = xcd_remap(blockIdx.x + nblk * blockIdx.y, nblk * splits);
   const int bid = lid % nblk, split = lid / nblk;
-  const int m_tile = bid % m_tiles, n_tile = bid / m_tiles;
+  int m_tile, n_tile;
+  tile_order(bid, m_tiles, n_tiles, kTileRowBlock, m_tile, n_tile);
   const int64_t M = p.m, N = p.n, K = p.k;
   const int64_t m0 = (int64_t)m_tile * BM, n0 = (int64_t)n_tile * (BN / NB);
   const int64_t kb = (int64_t)split * kchunk;
@@ -1201,7 +1212,8 @@ __global__ __launch_bounds__(64 * NWV, 1) void gemm_wide_kernel(GemmArgs p, int 
   const int nblk = m_tiles * n_tiles;
   const int lid = xcd_remap(blockIdx.x, nblk * splits);
   const int bid = lid % nblk, split = lid / nblk;
-  const int m_tile = bid % m_tiles, n_tile = bid / m_tiles;
+  int m_tile, n_tile;
+  tile_order(bid, m_tiles, n_tiles, kWideRowBlock, m_tile, n_tile);
   const int64_t M = p.m, N = p.n, K = p.k;
   const int64_t m0 = (int64_t)m_tile * kGwBM, n0 = (int64_t)n_tile * (GG ? 128 : 256);
   // K range [kb, kb + 64 nk) (splits > 1: PLAIN without rownorm, fp32
@@ -1508,7 +1520,8 @@ __global__ __launch_bounds__(256, 1) void gemm_wide_f8_kernel(GemmArgs p, int m_
   const int nblk = m_tiles * n_tiles;
   const int lid = xcd_remap(blockIdx.x, nblk * splits);
   const int bid = lid % nblk, split = lid / nblk;
-  const int m_tile = bid % m_tiles, n_tile = bid / m_tiles;
+  int m_tile, n_tile;
+  tile_order(bid, m_tiles, n_tiles, kWideRowBlock, m_tile, n_tile);
   const int64_t M = p.m, N = p.n, K = p.k;
   const int64_t m0 = (int64_t)m_tile * kGwBM, n0 = (int64_t)n_tile * (GG ? 128 : 256);
   // K range [kb, kb + 64 nk) (splits > 1: PLAIN without rownorm, partials
