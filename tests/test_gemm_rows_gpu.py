@@ -48,3 +48,71 @@ def test_geglu_row_blocks(m, fp8):
         got = K.gemm_geglu(x.cuda(), wg.cuda(), wu.cuda())
     g, u = x.float() @ wg.float().t(), x.float() @ wu.float().t()
     _close(got.cpu(), torch.nn.functional.gelu(g, approximate='tanh') * u)
+
+
+# gemm_pp_kernel: the sizes at which the plan takes its tiles of 256 x 128, 256 x
+# 192, 256 x 320 and 256 x 256 (the next test: 128 x 256), with rows and columns
+# one past a tile and ragged, and K with a partial last slab (k % 64 != 0); at
+# each size the operands that the epilogue build has.
+PP = [(6145, 1152, 712), (2000, 4000, 776), (6150, 1160, 456), (4111, 4304, 584),
+      (26000, 2048, 328), (6216, 2560, 712)]
+
+
+@pytest.mark.parametrize('m,n,k', PP)
+def test_pp_plain(m, n, k):
+    x, w = _rand((m, k), 11), _rand((n, k), 12, 0.05)
+    b, r, g = _rand((n,), 13), _rand((m, n), 14), _rand((m, n), 15)
+    got = K.gemm(x.cuda(), w.cuda(), bias=b.cuda(), residual=r.cuda(),
+                 gate=g.cuda(), act=2, rownorm_eps=1e-6)
+    xf = x.cuda().float()
+    xf = xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + 1e-6)
+    y = xf @ w.cuda().float().t() + b.cuda().float()
+    y = torch.nn.functional.gelu(y, approximate='tanh')
+    _close(got, y * g.cuda().float() + r.cuda().float())
+
+
+@pytest.mark.parametrize('m,n,k', [(6145, 1152, 712), (6528, 2560, 640),
+                                   (3000, 4104, 520)])
+def test_pp_row_sums_handed_on(m, n, k):
+    x, w, w2 = _rand((m, k), 21), _rand((n, k), 22, 0.05), _rand((k, n), 23, 0.02)
+    ss = torch.full((K.ss_parts(n), m), -1.0, device='cuda')
+    res = _rand((m, n), 24).cuda()
+    y = res.clone()
+    K.gemm(x.cuda(), w.cuda(), out=y, residual=y, ss_out=ss)
+    _close(y, x.cuda().float() @ w.cuda().float().t() + res.float())
+    pad = torch.nn.functional.pad(y.float().pow(2), (0, -n % 64))
+    blocks = pad.view(m, -1, 64).sum(-1).t()
+    # 64 squares summed in fp32 in another order
+    torch.testing.assert_close(ss, blocks, rtol=1e-5, atol=1e-5)
+    z = K.gemm(y, w2.cuda(), rownorm_eps=1e-6, ss_in=ss)
+    yf = y.float() * torch.rsqrt(y.float().pow(2).mean(-1, keepdim=True) + 1e-6)
+    _close(z, yf @ w2.cuda().float().t())
+
+
+@pytest.mark.parametrize('transposed', [True, False])
+@pytest.mark.parametrize('batch,seq,k', [(8, 777, 712), (31, 211, 520)])
+def test_pp_qkv_rope(batch, seq, k, transposed):
+    heads, hd = 8, 256
+    m, n, T = batch * seq, 2560, (seq + 10) // 8 * 8 + 8
+    x, w = _rand((m, k), 31).cuda(), _rand((n, k), 32, 0.05).cuda()
+    rope = K.rope_table(T, hd, device='cuda')
+    pos = torch.arange(seq, dtype=torch.int32, device='cuda').repeat(batch)
+    q = torch.zeros(m, heads * hd, dtype=BF16, device='cuda')
+    kc = torch.zeros(batch, T, hd, dtype=BF16, device='cuda')
+    vc = torch.zeros((batch, hd, T) if transposed else (batch, T, hd), dtype=BF16,
+                     device='cuda')
+    K.gemm_qkv_rope(x, w, rope, pos, q, kc.view(batch * T, hd),
+                    vc if transposed else vc.view(batch * T, hd), heads, hd,
+                    rownorm_eps=1e-6, row_group=seq, row_group_stride=T,
+                    v_ld=T if transposed else None)
+    xf = x.float() * torch.rsqrt(x.float().pow(2).mean(-1, keepdim=True) + 1e-6)
+    y = xf @ w.float().t()
+    c, s = rope[pos.long(), :, 0][:, None], rope[pos.long(), :, 1][:, None]
+    p = y[:, :(heads + 1) * hd].view(m, heads + 1, hd // 2, 2)
+    rot = torch.stack([p[..., 0] * c - p[..., 1] * s, p[..., 1] * c + p[..., 0] * s],
+                      -1).view(m, -1)
+    _close(q, rot[:, :heads * hd])
+    _close(kc[:, :seq].reshape(m, hd), rot[:, heads * hd:])
+    v = vc[:, :, :seq].transpose(1, 2) if transposed else vc[:, :seq]
+    _close(v.reshape(m, hd), y[:, (heads + 1) * hd:])
+    assert not kc[:, seq:].any()
