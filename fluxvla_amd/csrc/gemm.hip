@@ -2230,7 +2230,7 @@ using namespace fvx;
 extern "C" int64_t fvx_gemm_workspace_bytes(const fvx_gemm_desc* d) {
   if (!d || d->m <= 0) return 0;
   if (use_skinny(*d)) return plan_skinny(*d).ws_bytes;
-  if (plan_pp(*d) >= 0) return 0;
+  if (plan_mid(*d) >= 0 || plan_pp(*d) >= 0) return 0;
   // tiled path: fp32 partials (+ row sums) of every K split
   const int64_t sp = plan_tile(*d).splits;
   if (sp <= 1) return 0;
@@ -2319,6 +2319,8 @@ extern "C" int fvx_gemm(const fvx_gemm_desc* dp, void* stream) {
 #undef L
     return launch_status("gemm(skinny)");
   }
+  const int mid = plan_mid(d);
+  if (mid >= 0) return run_mid(d, mid, s);
   const int pp = plan_pp(d);
   if (pp >= 0) return run_pp(d, pp, s);
   TilePlan tp = plan_tile(d);

@@ -652,5 +652,8 @@ static bool a_grouped(const GemmArgs& d) { return d.a_row_group > 0 && d.m > d.a
 // serve it better or only they can) and its launch
 int plan_pp(const GemmArgs& d);
 int run_pp(const GemmArgs& d, int cfg, hipStream_t s);
+// gemm_mid.hip: the same for gemm_mid_kernel
+int plan_mid(const GemmArgs& d);
+int run_mid(const GemmArgs& d, int cfg, hipStream_t s);
 
 }  // namespace fvx

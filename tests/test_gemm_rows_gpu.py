@@ -90,8 +90,10 @@ def test_pp_row_sums_handed_on(m, n, k):
 
 
 @pytest.mark.parametrize('transposed', [True, False])
-@pytest.mark.parametrize('batch,seq,k', [(8, 777, 712), (31, 211, 520)])
-def test_pp_qkv_rope(batch, seq, k, transposed):
+# (gemm_pp_kernel twice, then gemm_mid_kernel's 128 x 128, 64 x 128 and 64 x 64)
+@pytest.mark.parametrize('batch,seq,k', [(8, 777, 712), (31, 211, 520), (2, 500, 200),
+                                         (8, 51, 136), (3, 47, 64)])
+def test_qkv_rope(batch, seq, k, transposed):
     heads, hd = 8, 256
     m, n, T = batch * seq, 2560, (seq + 10) // 8 * 8 + 8
     x, w = _rand((m, k), 31).cuda(), _rand((n, k), 32, 0.05).cuda()
@@ -116,3 +118,55 @@ def test_pp_qkv_rope(batch, seq, k, transposed):
     v = vc[:, :, :seq].transpose(1, 2) if transposed else vc[:, :seq]
     _close(v.reshape(m, hd), y[:, (heads + 1) * hd:])
     assert not kc[:, seq:].any()
+
+
+# gemm_mid_kernel: tiles of 64 x 64 and 64 x 128 over two K groups and of 128 x
+# 128, at the smallest and largest sizes of each, ragged rows and columns, an odd
+# number of slabs (one K group a slab short) and a partial last slab.
+MID = [(65, 64, 64), (65, 1160, 72), (408, 1024, 136), (1024, 1024, 200),
+       (70, 25608, 136), (769, 3456, 328), (2048, 2048, 64)]
+
+
+@pytest.mark.parametrize('rownorm', [False, True])
+@pytest.mark.parametrize('m,n,k', MID)
+def test_mid_plain(m, n, k, rownorm):
+    x, w = _rand((m, k), 41), _rand((n, k), 42, 0.05)
+    b, r, g = _rand((n,), 43), _rand((m, n), 44), _rand((m, n), 45)
+    got = K.gemm(x.cuda(), w.cuda(), bias=b.cuda(), residual=r.cuda(), act=1,
+                 gate=g.cuda(), rownorm_eps=1e-6 if rownorm else None)
+    xf = x.cuda().float()
+    if rownorm:
+        xf = xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + 1e-6)
+    y = torch.nn.functional.silu(xf @ w.cuda().float().t() + b.cuda().float())
+    _close(got, y * g.cuda().float() + r.cuda().float())
+
+
+@pytest.mark.parametrize('m,n,k', [(66, 72, 64), (816, 2048, 328), (1400, 2048, 264)])
+def test_mid_row_sums(m, n, k):
+    x, w, w2 = _rand((m, k), 51), _rand((n, k), 52, 0.05), _rand((2560, n), 53, 0.02)
+    ss0 = x.float().pow(2).sum(1)[None].cuda()
+    ss = torch.full((K.ss_parts(n), m), -1.0, device='cuda')
+    y = _rand((m, n), 54).cuda()
+    res = y.clone()
+    K.gemm(x.cuda(), w.cuda(), out=y, residual=y, rownorm_eps=1e-6, ss_in=ss0,
+           ss_out=ss)
+    xf = x.cuda().float()
+    xf = xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + 1e-6)
+    _close(y, xf @ w.cuda().float().t() + res.float())
+    pad = torch.nn.functional.pad(y.float().pow(2), (0, -n % 64))
+    # 64 squares summed in fp32 in another order
+    torch.testing.assert_close(ss, pad.view(m, -1, 64).sum(-1).t(), rtol=1e-5, atol=1e-5)
+    # more parts than the kernel keeps in registers
+    z = K.gemm(y, w2.cuda(), rownorm_eps=1e-6, ss_in=ss)
+    yf = y.float() * torch.rsqrt(y.float().pow(2).mean(-1, keepdim=True) + 1e-6)
+    _close(z, yf @ w2.cuda().float().t())
+
+
+@pytest.mark.parametrize('m,n,k', [(408, 4096, 200), (1281, 1480, 64), (129, 8200, 72)])
+def test_mid_geglu(m, n, k):
+    x, wg, wu = _rand((m, k), 61), _rand((n, k), 62, 0.1), _rand((n, k), 63, 0.1)
+    got = K.gemm_geglu(x.cuda(), wg.cuda(), wu.cuda(), rownorm_eps=1e-6)
+    xf = x.cuda().float()
+    xf = xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + 1e-6)
+    g = torch.nn.functional.gelu(xf @ wg.cuda().float().t(), approximate='tanh')
+    _close(got, g * (xf @ wu.cuda().float().t()))
