@@ -1962,7 +1962,7 @@ struct TilePlan {
   int cfg, splits;
 };
 
-// (After plan_pp, which serves most large bf16 PLAIN / QKV_ROPE problems.)
+// (After plan_mid and plan_pp, which serve most problems of many rows.)
 // The wide kernel (K % 64 == 0; PLAIN, GEGLU, fp8 QKV_ROPE) once its
 // 256 x 256 tiles number >= 256 (GEGLU) or, for PLAIN / QKV_ROPE, fill the
 // CUs (below) with K >= FVX_WIDE_MIN_K; config 1

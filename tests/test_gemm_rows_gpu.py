@@ -71,6 +71,43 @@ def test_pp_plain(m, n, k):
     _close(got, y * g.cuda().float() + r.cuda().float())
 
 
+# The same kernel with e4m3 weights (256 x 256 and 256 x 128 tiles; GeGLU 256 x
+# 2 x 128): rows and columns one past a tile and ragged, K of one and more pairs
+# of slabs; against the dequantized weights.
+@pytest.mark.parametrize('rownorm', [False, True])
+@pytest.mark.parametrize('m,n,k', [(6145, 1160, 1024), (2817, 2568, 2048), (6528, 2048, 2048),
+                                   (8190, 2040, 640)])
+def test_pp_fp8_plain(m, n, k, rownorm):
+    x, r, b = _rand((m, k), 71).cuda(), _rand((m, n), 72).cuda(), _rand((n,), 73).cuda()
+    w = K.Fp8Weight.quantize(_rand((n, k), 74, 0.05).cuda())
+    ss = torch.full((K.ss_parts(n), m), -1.0, device='cuda')
+    xf = x.float()
+    if rownorm:
+        xf = xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + 1e-6)
+    ref = xf @ w.dequantize().float().t()
+    got = K.gemm(x, w, bias=b, residual=r, rownorm_eps=1e-6 if rownorm else None)
+    _close(got, ref + b.float() + r.float())
+    y = r.clone()
+    K.gemm(x, w, out=y, residual=y, ss_out=ss, rownorm_eps=1e-6 if rownorm else None)
+    _close(y, ref + r.float())
+    pad = torch.nn.functional.pad(y.float().pow(2), (0, -n % 64))
+    # 64 squares summed in fp32 in another order
+    torch.testing.assert_close(ss, pad.view(m, -1, 64).sum(-1).t(), rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize('handed', [False, True])
+@pytest.mark.parametrize('m,n,k', [(257, 16384, 1024), (700, 16376, 2048), (1601, 4104, 1024)])
+def test_pp_fp8_geglu(m, n, k, handed):
+    x = _rand((m, k), 81).cuda()
+    wg = K.Fp8Weight.quantize(_rand((n, k), 82, 0.05).cuda())
+    wu = K.Fp8Weight.quantize(_rand((n, k), 83, 0.05).cuda())
+    ss = x.float().pow(2).sum(1)[None].contiguous() if handed else None
+    got = K.gemm_geglu(x, wg, wu, rownorm_eps=1e-6, ss_in=ss)
+    xf = x.float() * torch.rsqrt(x.float().pow(2).mean(-1, keepdim=True) + 1e-6)
+    g = torch.nn.functional.gelu(xf @ wg.dequantize().float().t(), approximate='tanh')
+    _close(got, g * (xf @ wu.dequantize().float().t()))
+
+
 @pytest.mark.parametrize('m,n,k', [(6145, 1152, 712), (6528, 2560, 640),
                                    (3000, 4104, 520)])
 def test_pp_row_sums_handed_on(m, n, k):
@@ -89,14 +126,19 @@ def test_pp_row_sums_handed_on(m, n, k):
     _close(z, yf @ w2.cuda().float().t())
 
 
+@pytest.mark.parametrize('fp8', [False, True])
 @pytest.mark.parametrize('transposed', [True, False])
 # (gemm_pp_kernel twice, then gemm_mid_kernel's 128 x 128, 64 x 128 and 64 x 64)
 @pytest.mark.parametrize('batch,seq,k', [(8, 777, 712), (31, 211, 520), (2, 500, 200),
                                          (8, 51, 136), (3, 47, 64)])
-def test_qkv_rope(batch, seq, k, transposed):
+def test_qkv_rope(batch, seq, k, transposed, fp8):
     heads, hd = 8, 256
     m, n, T = batch * seq, 2560, (seq + 10) // 8 * 8 + 8
+    if fp8:
+        k = -(-k // 128) * 128  # whole blocks of 128
     x, w = _rand((m, k), 31).cuda(), _rand((n, k), 32, 0.05).cuda()
+    if fp8:
+        w = K.Fp8Weight.quantize(w)
     rope = K.rope_table(T, hd, device='cuda')
     pos = torch.arange(seq, dtype=torch.int32, device='cuda').repeat(batch)
     q = torch.zeros(m, heads * hd, dtype=BF16, device='cuda')
@@ -108,7 +150,7 @@ def test_qkv_rope(batch, seq, k, transposed):
                     rownorm_eps=1e-6, row_group=seq, row_group_stride=T,
                     v_ld=T if transposed else None)
     xf = x.float() * torch.rsqrt(x.float().pow(2).mean(-1, keepdim=True) + 1e-6)
-    y = xf @ w.float().t()
+    y = xf @ (w.dequantize() if fp8 else w).float().t()
     c, s = rope[pos.long(), :, 0][:, None], rope[pos.long(), :, 1][:, None]
     p = y[:, :(heads + 1) * hd].view(m, heads + 1, hd // 2, 2)
     rot = torch.stack([p[..., 0] * c - p[..., 1] * s, p[..., 1] * c + p[..., 0] * s],
