@@ -19,8 +19,9 @@
 // and never produce NaN (a row that has seen no visible key yet keeps a zero
 // reference).  With kv_splits > 1 each split writes (O, m, l) partials to a
 // workspace and a merge kernel, the next kernel on the stream, combines them
-// in split order (deterministic).  This kernel serves SigLIP (head dim 72)
-// and any head dim other than 256 or a non-transposed V.  Head dim 256 with
+// in split order (deterministic).  This kernel serves any head dim other than
+// 256 or a non-transposed V; unmasked calls with one head per problem (SigLIP,
+// head dim 72) run attn_encoder_kernel (attention_encoder.hip).  Head dim 256 with
 // the transposed value cache runs attn_decode_kernel (the action expert: 408
 // query rows against the 867-key prefix+suffix cache, one 64-key tile per
 // workgroup) or attn_decode_t_kernel (the prefix prefill, key ranges of >= 4
@@ -31,6 +32,10 @@
 #include "common.h"
 
 namespace fvx {
+
+// attention_encoder.hip
+bool encoder_attn_ok(const fvx_attn_desc& d);
+int run_encoder_attn(const fvx_attn_desc& d, hipStream_t s);
 
 constexpr int kKeyTile = 64;
 constexpr float kLog2e = 1.4426950408889634f;
@@ -1543,6 +1548,7 @@ extern "C" int64_t fvx_attention_workspace_bytes(const fvx_attn_desc* d) {
   if (!d || d->sq <= 0 || d->sk <= 0 || d->heads <= 0 || d->n_problems <= 0)
     return 0;
   if (decode_ok(*d)) return plan_decode(*d).ws_bytes;
+  if (encoder_attn_ok(*d)) return 0;
   return plan_attn(*d).ws_bytes;
 }
 
@@ -1701,6 +1707,11 @@ extern "C" int fvx_attention(const fvx_attn_desc* dp, void* stream) {
                        dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s,
                        dk, a.n_rb, a.splits, dv);
     return launch_status("attention(decode merge)");
+  }
+  if (encoder_attn_ok(d)) {
+    FVX_REQUIRE(aligned16(d.workspace), FVX_ERR_ALIGN,
+                "attention: workspace must be 16B aligned");
+    return run_encoder_attn(d, s);
   }
   return run_generic(d, s);
 }

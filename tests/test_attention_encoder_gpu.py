@@ -1,0 +1,33 @@
+"""Unmasked attention with one query head per problem (the image encoder's), at
+the sizes where its kernel's two builds begin and end, and at sizes and scales
+that it leaves to the general kernel, against torch in fp32."""
+import pytest
+import torch
+
+from fluxvla_amd import kernels as K
+
+pytestmark = pytest.mark.gpu
+
+
+# 64 rows per workgroup up to 256 blocks of 64 rows (one per CU), then 128; one, an
+# odd and an even number of key tiles, ragged rows
+@pytest.mark.parametrize('n,sq,sk,hd', [
+    (1, 1, 64, 8), (3, 65, 128, 72), (2, 200, 192, 80), (48, 256, 256, 72),
+    (100, 130, 64, 40), (90, 257, 320, 72), (200, 130, 192, 80), (384, 256, 256, 72),
+    (256, 64, 64, 72), (257, 1, 64, 72),
+    # the general kernel: keys past the last whole tile
+    (3, 100, 100, 72)])
+def test_unmasked(n, sq, sk, hd):
+    g = torch.Generator().manual_seed(n + sq + sk + hd)
+    q, k, v = (torch.randn(n, s, hd, generator=g).to(torch.bfloat16).cuda()
+               for s in (sq, sk, sk))
+    q = q * 3  # a running maximum that moves
+    o = torch.full((n, sq + 1, hd), 7.0, dtype=torch.bfloat16, device='cuda')
+    for scale in (hd**-0.5, -0.1):  # (a negative scale: the general kernel)
+        K.mqa_attention(q, k, v, o[:, :sq], scale=scale)
+        s = torch.matmul(q.float(), k.float().transpose(1, 2).contiguous()) * scale
+        ref = torch.matmul(torch.softmax(s, -1), v.float())
+        # bf16 probabilities and output: 2^-8 of the largest value, four of them
+        err = (o[:, :sq].float() - ref).abs().max().item()
+        assert err <= 4 * 2.0**-8 * ref.abs().max().item(), (scale, err)
+        assert (o[:, sq:] == 7).all()
