@@ -337,11 +337,11 @@ def kernel_table(model):
     # to the next fused RMSNorm
     ss_a, ss_b = b['pre_ss'][0], b['pre_ss'][1]
     pre = [
-        ('gemm_tile_kernel<64,128,QKV_ROPE> (prefix)', lambda L: K.gemm_qkv_rope(
+        ('gemm_mid_kernel<128,128,QKV_ROPE> (prefix)', lambda L: K.gemm_qkv_rope(
             px, L['qkv_w'], model.rope, b['pos_pre'], b['pre_q'].view(M, -1),
             kc0.view(T, D), vc0, H, D, rownorm_eps=cfg.rms_eps, row_group=S,
             row_group_stride=T, v_ld=T, ss_in=ss_b), 2 * M * nq * cfg.llm_hidden),
-        ('gemm_tile_kernel<64,128,PLAIN> o-proj (prefix)', lambda L: K.gemm(
+        ('gemm_mid_kernel<64,128,PLAIN> 2 K groups, o-proj (prefix)', lambda L: K.gemm(
             b['pre_ctx'].view(M, -1), L['o_w'], out=b['pre_h'][:, :cfg.llm_hidden],
             residual=px, ss_out=ss_a), 2 * M * cfg.llm_hidden * H * D),
         ('gemm_wide_kernel<GEGLU> (prefix)', lambda L: K.gemm_geglu(
@@ -360,19 +360,19 @@ def kernel_table(model):
     Mv, vh = vx.shape
     nimg = Mv // cfg.num_patches
     vis = [
-        ('gemm_tile_kernel<64,128,PLAIN> qkv+bias (SigLIP)', lambda V: K.gemm(
+        ('gemm_mid_kernel<128,128,PLAIN> qkv+bias (SigLIP)', lambda V: K.gemm(
             vxn, V['qkv_w'], out=b['vis_qkv'], bias=V['qkv_b']),
          2 * Mv * 3 * vh * vh),
-        ('gemm_tile_kernel<64,64,PLAIN> o-proj+bias+res (SigLIP)',
+        ('gemm_mid_kernel<64,64,PLAIN> 2 K groups, o-proj+bias+res (SigLIP)',
          lambda V: K.gemm(b['vis_ctx'], V['o_w'], out=vxn, bias=V['o_b'],
                         residual=vx), 2 * Mv * vh * vh),
-        ('gemm_tile_kernel<64,128,PLAIN> fc1+bias+gelu (SigLIP)', lambda V: K.gemm(
+        ('gemm_mid_kernel<128,128,PLAIN> fc1+bias+gelu (SigLIP)', lambda V: K.gemm(
             vxn, V['fc1_w'], out=b['vis_h'], bias=V['fc1_b'], act=2),
          2 * Mv * cfg.vit_mlp * vh),
-        ('gemm_tile_kernel<64,64,PLAIN> fc2+bias+res (SigLIP)', lambda V: K.gemm(
+        ('gemm_mid_kernel<64,64,PLAIN> 2 K groups, fc2+bias+res (SigLIP)', lambda V: K.gemm(
             b['vis_h'], V['fc2_w'], out=vxn, bias=V['fc2_b'], residual=vx),
          2 * Mv * vh * cfg.vit_mlp),
-        ('attn_kernel<96,80> (SigLIP)', lambda V: K.mha_packed_qkv(
+        ('attn_encoder_kernel (SigLIP)', lambda V: K.mha_packed_qkv(
             b['vis_qkv'], b['vis_ctx'], nimg, cfg.num_patches, cfg.vit_heads,
             cfg.vit_head_dim),
          4 * nimg * cfg.vit_heads * cfg.num_patches ** 2 * cfg.vit_head_dim),
@@ -558,24 +558,24 @@ TABLE_DISPATCHES = (
     ('gemm_skinny_kernel<GEGLU> (expert)', [('gemm_skinny_kernel<1', 256, _E)]),
     ('gemm_skinny_kernel<PLAIN> down (expert)', [('gemm_skinny_kernel<0', 256, _E)]),
     ('attn_decode_kernel + merge (expert)', [('attn_decode_kernel', 176, _E)]),
-    ('gemm_tile_kernel<64,128,QKV_ROPE> (prefix)',
-     [('gemm_tile_kernel<64, 128, 2, 2, 3, 2', 260, _MP)]),
-    ('gemm_tile_kernel<64,128,PLAIN> o-proj (prefix)',
-     [('gemm_tile_kernel<64, 128, 2, 2, 4, 0', 208, _MP)]),
+    ('gemm_mid_kernel<128,128,QKV_ROPE> (prefix)',
+     [('gemm_mid_kernel<2, 1, 2, 4, 2', 140, _MP)]),
+    ('gemm_mid_kernel<64,128,PLAIN> 2 K groups, o-proj (prefix)',
+     [('gemm_mid_kernel<0, 1, 2, 2, 2', 208, _MP)]),
     ('gemm_wide_kernel<GEGLU> (prefix)', [('gemm_wide_kernel<1', 512, _MP)]),
     ('gemm_wide_kernel<PLAIN> 8 K ranges + split-K reduce, down (prefix)',
      [('gemm_wide_kernel<0', 256, _MP), ('gemm_partial_reduce_kernel<0', 816, _MP)]),
     ('attn_decode_t_kernel + merge (prefix)',
      [('attn_decode_t_kernel', 204, _MP), ('attn_decode_merge_kernel', 816, _MP)]),
-    ('gemm_tile_kernel<64,128,PLAIN> qkv+bias (SigLIP)',
-     [('gemm_tile_kernel<64, 128, 2, 2, 3, 0', 324, _MV)]),
-    ('gemm_tile_kernel<64,64,PLAIN> o-proj+bias+res (SigLIP)',
-     [('gemm_tile_kernel<64, 64, 2, 2, 4, 0', 216, _MV)]),
-    ('gemm_tile_kernel<64,128,PLAIN> fc1+bias+gelu (SigLIP)',
-     [('gemm_tile_kernel<64, 128, 2, 2, 3, 0', 408, _MV)]),
-    ('gemm_tile_kernel<64,64,PLAIN> fc2+bias+res (SigLIP)',
-     [('gemm_tile_kernel<64, 64, 2, 2, 4, 0', 216, _MV)]),
-    ('attn_kernel<96,80> (SigLIP)', [('attn_kernel<96, 80>', 192, _MV)]),
+    ('gemm_mid_kernel<128,128,PLAIN> qkv+bias (SigLIP)',
+     [('gemm_mid_kernel<0, 1, 2, 4, 2', 162, _MV)]),
+    ('gemm_mid_kernel<64,64,PLAIN> 2 K groups, o-proj+bias+res (SigLIP)',
+     [('gemm_mid_kernel<0, 1, 1, 2, 2', 216, _MV)]),
+    ('gemm_mid_kernel<128,128,PLAIN> fc1+bias+gelu (SigLIP)',
+     [('gemm_mid_kernel<0, 1, 2, 4, 2', 204, _MV)]),
+    ('gemm_mid_kernel<64,64,PLAIN> 2 K groups, fc2+bias+res (SigLIP)',
+     [('gemm_mid_kernel<0, 1, 1, 2, 2', 216, _MV)]),
+    ('attn_encoder_kernel (SigLIP)', [('attn_encoder_kernel', 192, _MV)]),
 )
 
 
