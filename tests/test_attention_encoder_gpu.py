@@ -31,3 +31,23 @@ def test_unmasked(n, sq, sk, hd):
         err = (o[:, :sq].float() - ref).abs().max().item()
         assert err <= 4 * 2.0**-8 * ref.abs().max().item(), (scale, err)
         assert (o[:, sq:] == 7).all()
+
+
+# the general kernel (kv_splits = 2) over the same operands: K, V and O as column
+# slices of wider rows, two problem strides, output rows of 8, 4 and 2 bytes'
+# alignment (the last one stays with the general kernel)
+@pytest.mark.parametrize('pad', [8, 4, 1])
+def test_matches_the_general_kernel(pad):
+    views, seq, heads, hd = 2, 192, 3, 72
+    hid = heads * hd
+    g = torch.Generator().manual_seed(pad)
+    qkv = torch.randn(views * seq, 3 * hid + 16, generator=g).to(torch.bfloat16).cuda()
+    outs = []
+    for splits in (0, 2):
+        o = torch.zeros(views * seq, hid + pad, dtype=torch.bfloat16, device='cuda')
+        K.mha_packed_qkv(qkv, o[:, :hid], views, seq, heads, hd, kv_splits=splits)
+        assert not o[:, hid:].any()
+        outs.append(o[:, :hid].float())
+    # bf16 probabilities and output on both sides: 2^-8 of the largest value each
+    err = (outs[0] - outs[1]).abs().max().item()
+    assert err <= 8 * 2.0**-8 * outs[1].abs().max().item(), err
