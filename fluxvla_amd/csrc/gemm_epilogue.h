@@ -151,7 +151,7 @@ __device__ __forceinline__ void bl_f8(__amdgpu_buffer_rsrc_t r, uint32_t off,
 // outside the item loops (an absent operand gets an empty view, whose reads
 // return zeros).
 struct EpiViews {
-  __amdgpu_buffer_rsrc_t bias, bf32, gate, res, pos, xt, prev, cw, rope, positions, csum;
+  __amdgpu_buffer_rsrc_t bias, bf32, bf32l, gate, res, pos, xt, prev, cw, rope, positions, csum;
 };
 
 // (SP: the plain-epilogue build -- PLAIN with bias, fp32 bias, activation,
@@ -161,7 +161,7 @@ template <int MODE, bool SP = false>
 __device__ __forceinline__ EpiViews epi_views(const GemmArgs& p) {
   EpiViews V;
   const int64_t N = p.n;
-  V.bias = V.bf32 = V.gate = V.res = V.pos = V.xt = V.prev = V.cw = V.rope = V.positions =
+  V.bias = V.bf32 = V.bf32l = V.gate = V.res = V.pos = V.xt = V.prev = V.cw = V.rope = V.positions =
       V.csum = make_rsrc(nullptr, 0u);
   if constexpr (SP) {
     V.bias = make_rsrc(p.bias, p.bias ? rec_bytes(N * 2) : 0u);
@@ -177,6 +177,7 @@ __device__ __forceinline__ EpiViews epi_views(const GemmArgs& p) {
   if (MODE == FVX_GEMM_PLAIN || MODE == FVX_GEMM_EULER) {
     V.bias = make_rsrc(p.bias, p.bias ? rec_bytes(N * 2) : 0u);
     V.bf32 = make_rsrc(p.bias_f32, p.bias_f32 ? rec_bytes(N * 4) : 0u);
+    V.bf32l = make_rsrc(p.bias_f32_locked, p.bias_f32_locked ? rec_bytes(N * 4) : 0u);
   }
   if (MODE == FVX_GEMM_EULER) {
     V.xt = make_rsrc(p.xt, rec_bytes(p.m * p.ldx * 4));
@@ -195,8 +196,6 @@ __device__ __forceinline__ EpiViews epi_views(const GemmArgs& p) {
   }
   return V;
 }
-
-__device__ __align__(16) const float kZeros8[8] = {};
 
 // the column operands of columns n .. n + 7 (bias_f32: the unlocked rows')
 // (LN: the kernel build with the folded LayerNorm, which reads ln_csum)
@@ -234,23 +233,11 @@ __device__ __forceinline__ void epi_load_row(const GemmArgs& p, const EpiViews& 
   const int rr = p.rtc_period > 0 ? (int)umod32(m, p.rtc_period) : 0;
   in.locked = false;
   if (p.rtc_lock) in.locked = rr < *(const __attribute__((address_space(4))) int32_t*)p.rtc_lock;
-  if (p.bias_f32_locked) {
-    // the row picks its fp32 bias array: a per-lane address, so global loads
-    // (a per-lane buffer view would loop over the lanes' views); an absent
-    // array or a column past cnt reads kZeros8
-    const float* b = in.locked ? p.bias_f32_locked : p.bias_f32;
-    if (vec) {
-      const f32x4_t* q = (const f32x4_t*)(b ? b + n : kZeros8);
-      const f32x4_t x0 = q[0], x1 = q[1];
+  if (p.bias_f32_locked) {  // (f0 holds the unlocked rows' bias: epi_load_col)
+    float fl[8];
+    bl_f8(V.bf32l, (uint32_t)(n * 4), vec, fl);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        in.f0[e] = x0[e];
-        in.f0[4 + e] = x1[e];
-      }
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) in.f0[e] = *(b && e < cnt ? b + n + e : kZeros8 + e);
-    }
+    for (int e = 0; e < 8; ++e) in.f0[e] = in.locked ? fl[e] : in.f0[e];
   }
   if (MODE == FVX_GEMM_EULER) {
     bl_f8(V.xt, (uint32_t)((m * p.ldx + n) * 4), vec, in.xt);

@@ -115,6 +115,28 @@ def test_plain_bias_f32_locked(K, cuda, m):
     assert rel_err(out, ref) <= 1e-2
 
 
+@pytest.mark.parametrize('m,n,k', [(100, 72, 64), (300, 1160, 128), (70, 3080, 136),
+                                   (100, 1160, 8192), (100, 1156, 64), (65, 8, 64)])
+def test_plain_bias_f32_locked_ragged(K, cuda, m, n, k):
+    """Columns past n in the last tile of the M > 64 kernels (one-round and tile
+    kernels): every operand is read through a view that ends at n, and what lies
+    behind the two bias arrays reaches no output."""
+    announce(f'gemm plain bias_f32_locked ragged {m} x {n} x {k}')
+    a, w = randn((m, k), 25), randn((n, k), 26, std=0.05)
+    both = torch.full((2, n + 256), float('nan'))
+    both[:, :n] = torch.randn(2, n, generator=gen(27))
+    dev = both.to(cuda)
+    lk = torch.tensor([9], dtype=torch.int32, device=cuda)
+    out = torch.full((m + 1, n + 8), 7.0, dtype=torch.bfloat16, device=cuda)
+    K.gemm(a.to(cuda), w.to(cuda), out=out[:m, :n], bias_f32=dev[0, :n],
+           bias_f32_locked=dev[1, :n], rtc_lock=lk, rtc_period=50)
+    locked = ((torch.arange(m) % 50) < 9)[:, None]
+    ref = a.float() @ w.float().t() + torch.where(locked, both[1, :n], both[0, :n])
+    # one bf16 rounding of each result
+    assert rel_err(out[:m, :n], ref) <= 4e-3
+    assert (out[m:] == 7).all() and (out[:, n:] == 7).all()
+
+
 def test_adarms_norm_locked(K, cuda):
     """Rows with row % 50 < lock take the locked style row (scale, shift
     and gate)."""
