@@ -433,7 +433,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void gemm_tile_kernel(
   // per wave); the shuffles run in every lane
   constexpr bool HO = MODE == FVX_GEMM_PLAIN && WNO == 64;
   const bool ho = HOX && HO && (p.ss_out || p.a8_out) && splits == 1;
-  const EpiViews V = epi_views<MODE, SP>(p);
+  const EpiViews V = epi_views<MODE, SP>(p, m0);
   // VA: every operand is 16B-aligned and N % 8 == 0 (uniform), so every
   // chunk with columns left holds 8 and moves as whole vectors
   auto epilogue = [&](auto va) {
@@ -734,7 +734,7 @@ __global__ __launch_bounds__(64 * NWV, 1) void gemm_wide_kernel(GemmArgs p, int 
   const int64_t nn = n0 + wn * WNO + 8 * ch;
   const int cnt = (int)(N - nn < 8 ? N - nn : 8);
   const bool ho = (MODE == FVX_GEMM_PLAIN || GG) && (p.ss_out || p.a8_out);
-  const EpiViews V = epi_views<MODE>(p);
+  const EpiViews V = epi_views<MODE>(p, m0);
   // block i of the accumulators -> scratch (compile-time indices, so the
   // accumulators stay in registers); the item loops below are real loops,
   // which keeps the epilogue code small enough for the kernel arguments to
@@ -1078,7 +1078,7 @@ __global__ __launch_bounds__(256, 1) void gemm_wide_f8_kernel(GemmArgs p, int m_
   const int64_t nn = n0 + wn * WNO + 8 * ch;
   const int cnt = (int)(N - nn < 8 ? N - nn : 8);
   const bool ho = (MODE == FVX_GEMM_PLAIN || GG) && (p.ss_out || p.a8_out);
-  const EpiViews V = epi_views<MODE>(p);
+  const EpiViews V = epi_views<MODE>(p, m0);
   auto to_scr = [&](auto ic) {
     constexpr int i = decltype(ic)::value;
 #pragma unroll
@@ -1421,7 +1421,7 @@ __global__ __launch_bounds__(64 * sk_waves(F8, A16)) void gemm_skinny_kernel(Gem
   const bool vec = vec_ok && cnt == 8;
   EpiIn in;
   if (mine) {
-    const EpiViews V = epi_views<MODE, SP>(p);
+    const EpiViews V = epi_views<MODE, SP>(p, 0);
     epi_load_col<MODE>(V, ncol, vec, in);
     epi_load_row<MODE, SP>(p, V, row, ncol, vec, cnt, in);
   }
@@ -1588,7 +1588,8 @@ __global__ __launch_bounds__(256) void gemm_partial_reduce_kernel(GemmArgs p,
       make_rsrc(ws, rec_bytes((NB * plane + (int64_t)splits * M) * 4));
   EpiIn in;
   {
-    const EpiViews V = epi_views<MODE, SP>(p);
+    // (the wave's first row: chunks, and so rows, rise with the lane)
+    const EpiViews V = epi_views<MODE, SP>(p, __builtin_amdgcn_readfirstlane((int)m));
     epi_load_col<MODE>(V, nn, vec_ok && cnt == 8, in);
     epi_load_row<MODE, SP>(p, V, m, nn, vec_ok && cnt == 8, cnt, in);
   }
@@ -1788,6 +1789,31 @@ static int validate(const GemmArgs& d) {
                   d.rtc_period < ((int64_t)1 << 31),
               FVX_ERR_SHAPE,
               "gemm: m, row_group, gate_group, pos_period and rtc_period must be < 2^31");
+  {
+    // the epilogue reads its row operands through one view per workgroup
+    // (epi_views): kEpiRows rows of each, or the whole operand, below 2 GiB
+    auto fits = [](int64_t total, int64_t tile, int64_t ld, int64_t size) {
+      return (total < tile ? total : tile) * ld * size < ((int64_t)1 << 31);
+    };
+    const int64_t rg = d.row_group, gg = d.gate_group > 1 ? d.gate_group : 1;
+    const int64_t last = d.m > 0 ? d.m - 1 : 0;
+    const int64_t orows = rg > 0 ? last / rg * d.row_group_stride + last % rg + 1 : d.m;
+    const int64_t otile =
+        rg > 0 ? (kEpiRows + rg - 2) / rg * d.row_group_stride + rg : kEpiRows;
+    const bool plain = d.mode == FVX_GEMM_PLAIN, euler = d.mode == FVX_GEMM_EULER;
+    FVX_REQUIRE(!plain || !d.residual || fits(orows, otile, d.ldr, 2), FVX_ERR_SHAPE,
+                "gemm: the residual rows of %lld product rows must span less than 2 GiB",
+                (long long)kEpiRows);
+    FVX_REQUIRE(!plain || !d.gate || fits((d.m + gg - 1) / gg, kEpiRows, d.ldg, 2),
+                FVX_ERR_SHAPE, "gemm: %lld gate rows must span less than 2 GiB",
+                (long long)kEpiRows);
+    FVX_REQUIRE(!plain || !d.pos || fits(d.pos_period, d.pos_period, d.ldp, 2), FVX_ERR_SHAPE,
+                "gemm: pos must be smaller than 2 GiB");
+    FVX_REQUIRE(!euler || (fits(d.m, kEpiRows, d.ldx, 4) &&
+                           (!d.rtc_prev || fits(d.m, kEpiRows, d.ld_prev, 4))),
+                FVX_ERR_SHAPE, "gemm(euler): %lld rows of xt and rtc_prev must span less than "
+                               "2 GiB", (long long)kEpiRows);
+  }
   switch (d.mode) {
     case FVX_GEMM_PLAIN:
       FVX_REQUIRE(d.c, FVX_ERR_NULL, "gemm: c is required");

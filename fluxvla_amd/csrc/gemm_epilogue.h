@@ -10,6 +10,9 @@ namespace fvx {
 
 typedef fvx_gemm_desc GemmArgs;
 
+// The largest number of product rows that one workgroup's epilogue covers
+constexpr int64_t kEpiRows = 256;
+
 // The first kCounterBytes of a GEMM workspace hold the per-column-tile
 // arrival counters of the split-K skinny kernel; fp32 partials follow.
 constexpr int kCounterBytes = 4096;
@@ -149,8 +152,12 @@ __device__ __forceinline__ void bl_f8(__amdgpu_buffer_rsrc_t r, uint32_t off,
 
 // Buffer views of the epilogue's operands: uniform, built once per wave
 // outside the item loops (an absent operand gets an empty view, whose reads
-// return zeros).
+// return zeros).  A view holds less than 2 GiB and its offsets have 32 bits, so
+// the row operands' views begin at the caller's first row m0 (m0, and below its
+// output and gate rows) and cover up to kEpiRows rows from there: operands of
+// any size are read right while those rows span less than 2 GiB (validate).
 struct EpiViews {
+  int64_t m0, orow0, grow0;
   __amdgpu_buffer_rsrc_t bias, bf32, bf32l, gate, res, pos, xt, prev, cw, rope, positions, csum;
 };
 
@@ -158,20 +165,23 @@ struct EpiViews {
 // a per-row gate, residual and the fragment-major copy only; the host
 // checks that the call uses nothing else)
 template <int MODE, bool SP = false>
-__device__ __forceinline__ EpiViews epi_views(const GemmArgs& p) {
+__device__ __forceinline__ EpiViews epi_views(const GemmArgs& p, int64_t m0) {
   EpiViews V;
-  const int64_t N = p.n;
+  const int64_t N = p.n, ml = p.m - m0;
+  V.m0 = V.orow0 = V.grow0 = m0;
   V.bias = V.bf32 = V.bf32l = V.gate = V.res = V.pos = V.xt = V.prev = V.cw = V.rope = V.positions =
       V.csum = make_rsrc(nullptr, 0u);
   if constexpr (SP) {
     V.bias = make_rsrc(p.bias, p.bias ? rec_bytes(N * 2) : 0u);
     V.bf32 = make_rsrc(p.bias_f32, p.bias_f32 ? rec_bytes(N * 4) : 0u);
-    V.res = make_rsrc(p.residual, p.residual ? rec_bytes(p.m * p.ldr * 2) : 0u);
-    V.gate = make_rsrc(p.gate, p.gate ? rec_bytes(p.m * p.ldg * 2) : 0u);
+    V.res = make_rsrc((const bf16_t*)p.residual + m0 * p.ldr,
+                      p.residual ? rec_bytes(ml * p.ldr * 2) : 0u);
+    V.gate = make_rsrc((const bf16_t*)p.gate + m0 * p.ldg,
+                       p.gate ? rec_bytes(ml * p.ldg * 2) : 0u);
     return V;
   }
   if (MODE == FVX_GEMM_QKV_ROPE) {
-    V.positions = make_rsrc(p.positions, rec_bytes(p.m * 4));
+    V.positions = make_rsrc(p.positions + m0, rec_bytes(ml * 4));
     V.rope = make_rsrc(p.rope, 0x7fffffffu);
   }
   if (MODE == FVX_GEMM_PLAIN || MODE == FVX_GEMM_EULER) {
@@ -180,17 +190,23 @@ __device__ __forceinline__ EpiViews epi_views(const GemmArgs& p) {
     V.bf32l = make_rsrc(p.bias_f32_locked, p.bias_f32_locked ? rec_bytes(N * 4) : 0u);
   }
   if (MODE == FVX_GEMM_EULER) {
-    V.xt = make_rsrc(p.xt, rec_bytes(p.m * p.ldx * 4));
-    V.prev = make_rsrc(p.rtc_prev, p.rtc_prev ? rec_bytes(p.m * p.ld_prev * 4) : 0u);
+    V.xt = make_rsrc(p.xt + m0 * p.ldx, rec_bytes(ml * p.ldx * 4));
+    V.prev = make_rsrc(p.rtc_prev + m0 * p.ld_prev,
+                       p.rtc_prev ? rec_bytes(ml * p.ld_prev * 4) : 0u);
     V.cw = make_rsrc(p.rtc_cw, p.rtc_cw ? rec_bytes(p.rtc_period * 4) : 0u);
   }
   if (MODE == FVX_GEMM_PLAIN) {
     V.csum = make_rsrc(p.ln_csum, p.ln_csum ? rec_bytes(N * 4) : 0u);
     const bool gdiv = p.gate_group > 1;
     const int64_t grows = gdiv ? udiv32(p.m + p.gate_group - 1, p.gate_group) : p.m;
-    V.gate = make_rsrc(p.gate, p.gate ? rec_bytes(grows * p.ldg * 2) : 0u);
-    V.res = make_rsrc(p.residual,
-                      p.residual ? rec_bytes((out_row(p, p.m - 1) + 1) * p.ldr * 2) : 0u);
+    V.grow0 = gdiv ? udiv32(m0, p.gate_group) : m0;
+    V.gate = make_rsrc((const bf16_t*)p.gate + V.grow0 * p.ldg,
+                       p.gate ? rec_bytes((grows - V.grow0) * p.ldg * 2) : 0u);
+    // (from the start of m0's group: no row of the tile lies before it)
+    if (p.row_group > 0) V.orow0 = (int64_t)udiv32(m0, p.row_group) * p.row_group_stride;
+    V.res = make_rsrc((const bf16_t*)p.residual + V.orow0 * p.ldr,
+                      p.residual ? rec_bytes((out_row(p, p.m - 1) + 1 - V.orow0) * p.ldr * 2)
+                                 : 0u);
     const int64_t pp = p.pos_period > 0 ? p.pos_period : 1;
     V.pos = make_rsrc(p.pos, p.pos ? rec_bytes(pp * p.ldp * 2) : 0u);
   }
@@ -214,16 +230,17 @@ __device__ __forceinline__ void epi_load_row(const GemmArgs& p, const EpiViews& 
                                              int64_t n, bool vec, int cnt, EpiIn& in) {
   if (MODE == FVX_GEMM_GEGLU) return;
   if constexpr (SP) {
-    // 32-bit offsets: the host keeps m * ldr and m * ldg below 2^31
-    in.res = bl_b8(V.res, ((uint32_t)m * (uint32_t)p.ldr + (uint32_t)n) * 2u, vec);
-    in.gate = bl_b8(V.gate, ((uint32_t)m * (uint32_t)p.ldg + (uint32_t)n) * 2u, vec);
+    const uint32_t ml = (uint32_t)m - (uint32_t)V.m0;
+    in.res = bl_b8(V.res, (ml * (uint32_t)p.ldr + (uint32_t)n) * 2u, vec);
+    in.gate = bl_b8(V.gate, (ml * (uint32_t)p.ldg + (uint32_t)n) * 2u, vec);
     return;
   }
   if (MODE == FVX_GEMM_QKV_ROPE) {
     const int hd = p.head_dim;
     const bool rot = n < (int64_t)(p.n_q_heads + 1) * hd;
     const int64_t pos =
-        (int32_t)__builtin_amdgcn_raw_buffer_load_b32(V.positions, (uint32_t)(m * 4), 0, 0);
+        (int32_t)__builtin_amdgcn_raw_buffer_load_b32(V.positions, (uint32_t)((m - V.m0) * 4),
+                                                      0, 0);
     bl_f8(V.rope, rot ? (uint32_t)((pos * (hd >> 1) + (umod32(n, hd) >> 1)) * 8) : kOOB, vec,
           in.f0);
     return;
@@ -240,14 +257,14 @@ __device__ __forceinline__ void epi_load_row(const GemmArgs& p, const EpiViews& 
     for (int e = 0; e < 8; ++e) in.f0[e] = in.locked ? fl[e] : in.f0[e];
   }
   if (MODE == FVX_GEMM_EULER) {
-    bl_f8(V.xt, (uint32_t)((m * p.ldx + n) * 4), vec, in.xt);
-    bl_f8(V.prev, (uint32_t)((m * p.ld_prev + n) * 4), vec, in.prev);
+    bl_f8(V.xt, (uint32_t)(((m - V.m0) * p.ldx + n) * 4), vec, in.xt);
+    bl_f8(V.prev, (uint32_t)(((m - V.m0) * p.ld_prev + n) * 4), vec, in.prev);
     in.cw = bload1f(V.cw, (uint32_t)(rr * 4));
     return;
   }
-  in.gate = bl_b8(V.gate, (uint32_t)(((p.gate_group > 1 ? udiv32(m, p.gate_group) : m) * p.ldg + n) * 2),
-                  vec);
-  in.res = bl_b8(V.res, (uint32_t)((out_row(p, m) * p.ldr + n) * 2), vec);
+  const int64_t grow = (p.gate_group > 1 ? udiv32(m, p.gate_group) : m) - V.grow0;
+  in.gate = bl_b8(V.gate, (uint32_t)((grow * p.ldg + n) * 2), vec);
+  in.res = bl_b8(V.res, (uint32_t)(((out_row(p, m) - V.orow0) * p.ldr + n) * 2), vec);
   in.pos = bl_b8(V.pos,
                  (uint32_t)(((p.pos_period > 1 ? umod32(m, p.pos_period) : 0) * p.ldp + n) * 2),
                  vec);
@@ -624,12 +641,11 @@ static bool epi_vec_ok(const GemmArgs& d) {
 // kernel's XF bit 3, the skinny kernel's and the split-K reduce's SP)?
 // Bias, fp32 bias, activation, a per-row gate, residual, the fragment-major
 // copy, the fused RMSNorm and the hand-overs only, bf16 output rows below
-// 2^31 elements from the start of c, of the residual and of the gate.
+// 2^31 elements from the start of c.
 static bool plain_epilogue_ok(const GemmArgs& d) {
   return d.mode == FVX_GEMM_PLAIN && !d.pos && !d.out_f32 && d.row_group == 0 && !d.rtc_lock &&
          !d.bias_f32_locked && !d.ln_csum && d.m * d.ldc < ((int64_t)1 << 31) &&
-         (!d.residual || d.m * d.ldr < ((int64_t)1 << 31)) &&
-         (!d.gate || (d.gate_group <= 1 && d.m * d.ldg < ((int64_t)1 << 31)));
+         (!d.gate || d.gate_group <= 1);
 }
 
 // A's rows in groups with gaps between them (fvx_gemm_desc.a_row_group)

@@ -105,7 +105,7 @@ __global__ __launch_bounds__(512, 1) void gemm_mid_kernel(GemmArgs p, int m_tile
   auto n_of = [&](int j, int h) {
     return n0 + 32 * (JO * wn + j) + 16 * (KG == 2 ? kg : h) + 8 * hk;
   };
-  const EpiViews V = epi_views<MODE, SP>(p);
+  const EpiViews V = epi_views<MODE, SP>(p, m0);
   EpiIn in[RB][JO][HN];
   // the epilogue's operands and the handed-over row sums, behind the first slabs
 #pragma unroll

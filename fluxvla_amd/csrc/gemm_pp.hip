@@ -244,7 +244,7 @@ __global__ __launch_bounds__(512, 1) void gemm_pp_kernel(GemmArgs p, int m_tiles
   // >> 2) + 4 hk + (r & 3) of 32 j; chunk h of it, columns 16 h + 8 hk .. + 7,
   // after the half-waves swap.  N % 8 == 0 and 16-byte operands (the host
   // checks): every chunk with columns left moves whole.
-  const EpiViews V = epi_views<MODE, SP>(p);
+  const EpiViews V = epi_views<MODE, SP>(p, m0);
   const __amdgpu_buffer_rsrc_t rs0 = make_rsrc(p.b_scale, F8 ? rec_bytes(p.n * 4) : 0u);
   const __amdgpu_buffer_rsrc_t rs1 =
       make_rsrc(p.b2_scale, F8 && NB == 2 ? rec_bytes(p.n * 4) : 0u);

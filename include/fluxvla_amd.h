@@ -72,6 +72,10 @@ enum fvx_act { FVX_ACT_NONE = 0, FVX_ACT_SILU = 1, FVX_ACT_GELU_TANH = 2 };
  * (identity when row_group == 0).  m, row_group, gate_group, pos_period and
  * rtc_period must be below 2^31 (FVX_ERR_SHAPE otherwise): the epilogue
  * divides by them in 32 bits.
+ * Operands may be larger than 2 GiB, but the rows of residual, gate (PLAIN),
+ * xt and rtc_prev (EULER) that 256 consecutive product rows use, and all of
+ * pos, must each span less (FVX_ERR_SHAPE otherwise): one workgroup reads them
+ * through one view.
  */
 typedef struct fvx_gemm_desc {
   const void* a; int64_t lda;      /* [M, K] bf16 */

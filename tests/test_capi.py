@@ -95,6 +95,25 @@ def test_gemm_rejects_periods_past_32_bits():
         assert '2^31' in _err(lib)
 
 
+def test_gemm_rejects_epilogue_rows_past_a_view():
+    # 256 rows of a row operand are read through one view below 2 GiB
+    lib = _lib.load()
+    ld = (1 << 22) + 8
+    for kw in ({'residual': 65536, 'ldr': ld}, {'gate': 65536, 'ldg': ld, 'gate_group': 1},
+               {'residual': 65536, 'ldr': 64, 'row_group': 1, 'row_group_stride': 1 << 17},
+               {'pos': 65536, 'ldp': ld, 'pos_period': 300},
+               {'mode': _lib.GEMM_EULER, 'xt': 65536, 'ldx': ld // 2},
+               {'mode': _lib.GEMM_EULER, 'xt': 65536, 'ldx': 64, 'rtc_prev': 65536,
+                'ld_prev': ld // 2, 'rtc_period': 50, 'rtc_lock': 4096}):
+        d = _lib.GemmDesc()
+        d.a, d.b, d.c = 4096, 8192, 16384
+        d.m, d.n, d.k, d.lda, d.ldb, d.ldc = 300, 64, 64, 64, 64, 64
+        for k, v in kw.items():
+            setattr(d, k, v)
+        assert lib.fvx_gemm(ctypes.byref(d), None) == _lib.FVX_ERR_SHAPE, kw
+        assert '2 GiB' in _err(lib), kw
+
+
 def test_gemm_rejects_bad_layernorm_fold():
     # ln_csum: PLAIN, rownorm, M > 64, sums taken in the K loop (no ss_in),
     # bf16 weights, one K range, nothing handed over
