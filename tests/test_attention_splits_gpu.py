@@ -58,3 +58,23 @@ def test_default_splits_fit_the_workspace(keep):
     d.workspace_bytes = int(need * keep)
     K.run_attention(d)
     _check(o, ref)
+
+
+def test_more_splits_than_the_merge_addresses():
+    """65100 key splits asked for: 4.3 GB of partials, more than 32-bit offsets reach."""
+    sk, hd, splits = 65100 * 64, 256, 65100
+    q = torch.zeros(1, 1, hd, dtype=BF16, device='cuda')
+    k = torch.zeros(1, sk, hd, dtype=BF16, device='cuda')  # equal scores: the mean of v
+    v = (torch.arange(sk, device='cuda') % 512 / 256.0).to(BF16)[None, :, None].expand(
+        1, sk, hd).contiguous()
+    o = torch.zeros_like(q)
+    d = K.attention_desc(q, k, v, o, sq=1, sk=sk, heads=1, head_dim=hd, q_tok_stride=hd,
+                         q_head_stride=hd, k_tok_stride=hd, v_tok_stride=hd,
+                         o_tok_stride=hd, o_head_stride=hd, kv_splits=splits)
+    need = _lib.load().fvx_attention_workspace_bytes(ctypes.byref(d))
+    ws = torch.zeros(need, dtype=torch.uint8, device='cuda')
+    d.workspace, d.workspace_bytes = ws.data_ptr(), need
+    K.run_attention(d)
+    # bf16 probabilities (exactly 1) and output: one rounding of the mean
+    ref = v[0, :, 0].double().mean().item()
+    assert (o.double() - ref).abs().max().item() <= 2.0**-8 * ref
