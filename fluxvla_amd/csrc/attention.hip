@@ -328,14 +328,14 @@ __device__ __forceinline__ void store_rows(const fvx_attn_desc& p, bf16_t* O,
 
 // Combine the split partials of one row block (same lane layout as the
 // attention kernel): global max, rescale, sum, in split order.  A workgroup
-// takes one 16-dim fragment (blockIdx.y) of the 64 rows, with up to 16 splits'
-// loads in flight: one workgroup for all 256 dims left 7 CUs to read the 3 MB of
+// takes one 16-dim fragment (blockIdx.y) of the 64 rows, with NS splits' loads in
+// flight: one workgroup for all 256 dims left 7 CUs to read the 3 MB of
 // partials of the 400-row decode (20.9 us per call, now 6.8).
-template <int HDP, int HDV>
+template <int HDP, int HDV, int NS>
 __global__ __launch_bounds__(256) void attn_merge_kernel(fvx_attn_desc p,
                                                          int n_row_blocks,
                                                          int splits) {
-  constexpr int ND = HDV / 16, NS = 16;
+  constexpr int ND = HDV / 16;
   constexpr int64_t PF = attn_part_floats<HDP, HDV>();
   warm_kernargs<sizeof(fvx_attn_desc) + 8>();
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -1599,14 +1599,28 @@ static int run_generic(const fvx_attn_desc& d, hipStream_t s) {
                        a.n_row_blocks, a.splits, a.kps);
   int st = launch_status("attention");
   if (st || a.splits == 1) return st;
+  // The merge's loads in flight: the smallest build that holds all splits in one
+  // pass.  Two or three splits over many row blocks wait for the loads past them
+  // (us per call, 8 x 100 rows x 8 heads, 500 keys in 2 splits: one build of 16 37.2,
+  // this 32.5, a workgroup for all 256 dims 35.3; 1 x 100 rows, 866 keys: 21.7, 19.3,
+  // 34.8; 50 rows, 866 keys in 14: 17.6, 17.6, 33.3).
   const unsigned frags = a.hdp == 256 ? 16u : 5u;
   dim3 mgrid((unsigned)a.n_row_blocks, frags, (unsigned)d.n_problems);
-  if (a.hdp == 256)
-    hipLaunchKernelGGL((attn_merge_kernel<256, 256>), mgrid, dim3(256), 0, s,
-                       dk, a.n_row_blocks, a.splits);
+  auto merge = [&](auto ns) {
+    constexpr int NS = decltype(ns)::value;
+    if (a.hdp == 256)
+      hipLaunchKernelGGL((attn_merge_kernel<256, 256, NS>), mgrid, dim3(256), 0, s, dk,
+                         a.n_row_blocks, a.splits);
+    else
+      hipLaunchKernelGGL((attn_merge_kernel<96, 80, NS>), mgrid, dim3(256), 0, s, dk,
+                         a.n_row_blocks, a.splits);
+  };
+  if (a.splits <= 4)
+    merge(IntC<4>{});
+  else if (a.splits <= 8)
+    merge(IntC<8>{});
   else
-    hipLaunchKernelGGL((attn_merge_kernel<96, 80>), mgrid, dim3(256), 0, s, dk,
-                       a.n_row_blocks, a.splits);
+    merge(IntC<16>{});
   return launch_status("attention");
 }
 

@@ -42,6 +42,16 @@ def test_splits(sq, sk, heads, hd, splits):
     _check(o, ref)
 
 
+# the merge's builds of 4, 8 and 16 splits a pass, from their first to their last
+@pytest.mark.parametrize('splits', [3, 4, 5, 8, 9])
+@pytest.mark.parametrize('sq,sk,heads,hd', [(67, 4600, 2, 256), (70, 4600, 3, 72)])
+def test_merge_builds(sq, sk, heads, hd, splits):
+    (q, k, v, kg, qg), ref = _inputs(sq, sk, heads, hd)
+    o = torch.zeros_like(q)
+    K.mqa_attention(q, k, v, o, kgrp=kg, qgrp=qg, kv_splits=splits)
+    _check(o, ref)
+
+
 @pytest.mark.parametrize('keep', [0.0, 0.4, 1.0])
 def test_default_splits_fit_the_workspace(keep):
     """With less workspace than the default plan wants, fewer splits."""
