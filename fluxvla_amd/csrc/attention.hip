@@ -1454,7 +1454,11 @@ static AttnPlan plan_attn(const fvx_attn_desc& d) {
     // one 64-key tile per split for head dim 256 (the decode with row-major
     // values, 400 rows x 866 keys: 14 splits against 7, 15.9 -> 11.0 us),
     // two otherwise
-    const int64_t max_split = a.hdp == 256 ? (d.sk + 63) / 64 : (d.sk + 127) / 128;
+    int64_t max_split = a.hdp == 256 ? (d.sk + 63) / 64 : (d.sk + 127) / 128;
+    // Two tiles: the second workgroup saves 4 us and its merge costs more with many
+    // row blocks (one split / two: 25 row blocks 14.6 / 13.7, 32 14.6 / 12.1, 56
+    // 14.8 / 16.7, 80 14.8 / 18.8, 104 15.1 / 21.6).
+    if (max_split == 2 && a.hdp == 256 && blocks > 32) max_split = 1;
     if (splits > max_split) splits = (int)max_split;
     if (splits > 32) splits = 32;
     if (splits < 1) splits = 1;

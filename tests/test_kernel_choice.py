@@ -1,0 +1,37 @@
+"""Which kernel, and how many key ranges, a call takes: the rules of the dispatch as
+its workspace query shows them (no GPU needed; 256 CUs are assumed without one)."""
+import ctypes
+
+import pytest
+
+from fluxvla_amd import _lib
+
+
+def _attn(rows, sk, head_dim, heads=1, problems=1, **kw):
+    d = _lib.AttnDesc()
+    d.q, d.k, d.v, d.o = 4096, 8192, 16384, 32768
+    d.sq, d.sk, d.heads, d.head_dim, d.n_problems, d.zdiv = rows, sk, heads, head_dim, problems, 1
+    d.q_tok_stride = d.o_tok_stride = heads * head_dim
+    d.q_head_stride = d.o_head_stride = d.k_tok_stride = d.v_tok_stride = head_dim
+    d.scale = head_dim**-0.5
+    for k, v in kw.items():
+        setattr(d, k, v)
+    return d
+
+
+def _splits(d):
+    """Key ranges: the workspace holds 64 KiB of counters and the partials."""
+    ws = _lib.load().fvx_attention_workspace_bytes(ctypes.byref(d))
+    if not ws:
+        return 1
+    dims = 256 if d.head_dim > 80 else 80
+    blocks = -(-d.sq * d.heads // 64) * d.n_problems
+    return (ws - 65536) // (blocks * (64 * dims + 128) * 4)
+
+
+# two tiles are split for up to 32 blocks of 64 rows, more tiles at every size
+@pytest.mark.parametrize('rows,problems,sk,splits', [
+    (50, 1, 64, 1), (50, 1, 65, 2), (50, 1, 128, 2), (256, 1, 128, 2), (257, 1, 128, 1),
+    (50, 8, 128, 1), (50, 8, 129, 3), (100, 8, 100, 1), (100, 8, 192, 2), (50, 1, 866, 14)])
+def test_row_major_head_dim_256(rows, problems, sk, splits):
+    assert _splits(_attn(rows, sk, 256, heads=8, problems=problems)) == splits
