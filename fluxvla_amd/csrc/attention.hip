@@ -21,7 +21,8 @@
 // workspace and a merge kernel, the next kernel on the stream, combines them
 // in split order (deterministic).  This kernel serves any head dim other than
 // 256 or a non-transposed V; unmasked calls with one head per problem (SigLIP,
-// head dim 72) run attn_encoder_kernel (attention_encoder.hip).  Head dim 256 with
+// head dim 72) run attn_encoder_kernel (attention_encoder.hip) unless splitting
+// their keys is faster (encoder_first).  Head dim 256 with
 // the transposed value cache runs attn_decode_kernel (the action expert: 408
 // query rows against the 867-key prefix+suffix cache, one 64-key tile per
 // workgroup) or attn_decode_t_kernel (the prefix prefill, key ranges of >= 4
@@ -1554,12 +1555,40 @@ static bool decode_ok(const fvx_attn_desc& d) {
   return use_decode(d) && dec_div_exact(d, plan_decode(d));
 }
 
+// With automatic splits (kv_splits <= 0) and less workspace than they need: as many
+// as it holds.
+static AttnPlan plan_attn_fitting(const fvx_attn_desc& d) {
+  const AttnPlan a = plan_attn(d);
+  if (a.splits == 1 || d.kv_splits > 1 || (d.workspace && d.workspace_bytes >= a.ws_bytes))
+    return a;
+  const int64_t per = (a.ws_bytes - kAttnCounterBytes) / a.splits;
+  const int64_t fit = d.workspace ? (d.workspace_bytes - kAttnCounterBytes) / per : 0;
+  fvx_attn_desc t = d;
+  t.kv_splits = fit >= 2 && d.kv_splits <= 0 ? (int)fit : 1;
+  return plan_attn(t);
+}
+
+// attn_encoder_kernel where it can serve d, or attn_kernel over the plan's key
+// ranges and the merge: the encoder kernel walks all T key tiles in one workgroup
+// and takes about 2.8 + 0.93 T us while 64-row blocks have a CU each, attn_kernel
+// with ranges of t tiles and its merge 6.1 to 7.4 + 2.1 t with 1 to 32 blocks (and more
+// past them).
+// Measured (us, encoder / general; head dim 72, blocks of 64 rows x tiles): 1 x 8
+// 10.1 / 10.1, 1 x 16 17.7 / 10.4, 1 x 64 61.9 / 17.3; 16 x 8 10.3 / 10.8, 16 x 12
+// 14.1 / 11.4, 48 x 10 12.4 / 14.0, 48 x 24 25.6 / 20.9; 64 x 20 21.8 / 23.3, 64 x 32
+// 36.0 / 32.3; 80 x 96 (two ranges) 101 / 110.
+static bool encoder_first(const fvx_attn_desc& d, const AttnPlan& a) {
+  const int64_t tiles = d.sk / kKeyTile, range = a.kps / kKeyTile;
+  const int64_t blocks = (int64_t)a.n_row_blocks * d.n_problems;
+  return encoder_attn_ok(d) && 4 * tiles <= 14 + (blocks < 32 ? blocks : 32) / 8 + 9 * range;
+}
+
 extern "C" int64_t fvx_attention_workspace_bytes(const fvx_attn_desc* d) {
   if (!d || d->sq <= 0 || d->sk <= 0 || d->heads <= 0 || d->n_problems <= 0)
     return 0;
   if (decode_ok(*d)) return plan_decode(*d).ws_bytes;
-  if (encoder_attn_ok(*d)) return 0;
-  return plan_attn(*d).ws_bytes;
+  const AttnPlan a = plan_attn(*d);
+  return encoder_first(*d, a) ? 0 : a.ws_bytes;
 }
 
 // The descriptor the kernels see: the split partials start past the arrival
@@ -1576,20 +1605,11 @@ static fvx_attn_desc past_counters(const fvx_attn_desc& d) {
   return k;
 }
 
-static int run_generic(const fvx_attn_desc& d, hipStream_t s) {
-  AttnPlan a = plan_attn(d);
-  if (a.splits > 1 && (!d.workspace || d.workspace_bytes < a.ws_bytes)) {
-    FVX_REQUIRE(d.kv_splits <= 1, FVX_ERR_WORKSPACE,
-                "attention: kv_splits=%d needs %lld workspace bytes, got %lld",
-                d.kv_splits, (long long)a.ws_bytes,
-                (long long)d.workspace_bytes);
-    // as many splits as the workspace holds
-    const int64_t per = (a.ws_bytes - kAttnCounterBytes) / a.splits;
-    const int64_t fit = d.workspace ? (d.workspace_bytes - kAttnCounterBytes) / per : 0;
-    fvx_attn_desc t = d;
-    t.kv_splits = fit >= 2 && d.kv_splits <= 0 ? (int)fit : 1;
-    a = plan_attn(t);
-  }
+static int run_generic(const fvx_attn_desc& d, const AttnPlan& a, hipStream_t s) {
+  FVX_REQUIRE(a.splits == 1 || (d.workspace && d.workspace_bytes >= a.ws_bytes),
+              FVX_ERR_WORKSPACE,
+              "attention: kv_splits=%d needs %lld workspace bytes, got %lld",
+              d.kv_splits, (long long)a.ws_bytes, (long long)d.workspace_bytes);
   FVX_REQUIRE(aligned16(d.workspace), FVX_ERR_ALIGN,
               "attention: workspace must be 16B aligned");
   const fvx_attn_desc dk = past_counters(d);
@@ -1732,12 +1752,13 @@ extern "C" int fvx_attention(const fvx_attn_desc* dp, void* stream) {
                        dk, a.n_rb, a.splits, dv);
     return launch_status("attention(decode merge)");
   }
-  if (encoder_attn_ok(d)) {
+  const AttnPlan a = plan_attn_fitting(d);
+  if (encoder_first(d, a)) {
     FVX_REQUIRE(aligned16(d.workspace), FVX_ERR_ALIGN,
                 "attention: workspace must be 16B aligned");
     return run_encoder_attn(d, s);
   }
-  return run_generic(d, s);
+  return run_generic(d, a, s);
 }
 // Zeroes the attention workspace's counter region (a fill kernel, not a
 // memset node: callers may run it next to captured work).

@@ -51,3 +51,30 @@ def test_matches_the_general_kernel(pad):
     # bf16 probabilities and output on both sides: 2^-8 of the largest value each
     err = (outs[0] - outs[1]).abs().max().item()
     assert err <= 8 * 2.0**-8 * outs[1].abs().max().item(), err
+
+
+# few rows and many keys: split keys and the merge with the default's workspace, the
+# unsplit walk with none and with one range asked for
+@pytest.mark.parametrize('ws,splits', [(None, 0), (0, 0), (None, 1)])
+@pytest.mark.parametrize('n,sq,sk,hd', [(1, 64, 4096, 72), (4, 64, 1024, 72), (2, 7, 640, 80),
+                                        (48, 64, 896, 40)])
+def test_few_rows_many_keys(n, sq, sk, hd, ws, splits):
+    g = torch.Generator().manual_seed(n + sq + sk + hd)
+    q, k, v = (torch.randn(n, s, hd, generator=g).to(torch.bfloat16).cuda()
+               for s in (sq, sk, sk))
+    q = q * 3  # a running maximum that moves
+    o = torch.full((n, sq + 1, hd), 7.0, dtype=torch.bfloat16, device='cuda')
+    d = K.attention_desc(q, k, v, o, sq=sq, sk=sk, heads=1, head_dim=hd, n_problems=n,
+                         q_tok_stride=hd, q_head_stride=hd, q_zs=(sq * hd, 0),
+                         k_tok_stride=hd, k_zs=(sk * hd, 0), v_tok_stride=hd,
+                         v_zs=(sk * hd, 0), o_tok_stride=hd, o_head_stride=hd,
+                         o_zs=((sq + 1) * hd, 0), kv_splits=splits)
+    if ws is not None:
+        d.workspace, d.workspace_bytes = None, ws
+    K.run_attention(d)
+    s = torch.matmul(q.float(), k.float().transpose(1, 2).contiguous()) * hd**-0.5
+    ref = torch.matmul(torch.softmax(s, -1), v.float())
+    # bf16 probabilities and output: 2^-8 of the largest value, four of them
+    err = (o[:, :sq].float() - ref).abs().max().item()
+    assert err <= 4 * 2.0**-8 * ref.abs().max().item(), err
+    assert (o[:, sq:] == 7).all()

@@ -35,3 +35,17 @@ def _splits(d):
     (50, 8, 128, 1), (50, 8, 129, 3), (100, 8, 100, 1), (100, 8, 192, 2), (50, 1, 866, 14)])
 def test_row_major_head_dim_256(rows, problems, sk, splits):
     assert _splits(_attn(rows, sk, 256, heads=8, problems=problems)) == splits
+
+
+# unmasked, one head: few blocks of 64 rows over many key tiles are split, short walks
+# and problems that fill the CUs are not
+@pytest.mark.parametrize('rows,problems,tiles,splits', [
+    (64, 1, 8, 1), (64, 1, 9, 5), (64, 31, 9, 5), (64, 32, 9, 1), (64, 32, 10, 5),
+    (64, 1, 64, 32), (1, 1, 64, 32), (64, 4, 16, 8), (64, 16, 8, 1),
+    (256, 16, 4, 1), (64, 48, 11, 1), (64, 48, 14, 4), (64, 64, 20, 1), (64, 64, 32, 3),
+    (64, 80, 96, 1), (256, 64, 64, 1)])
+def test_unmasked_one_head(rows, problems, tiles, splits):
+    assert _splits(_attn(rows, 64 * tiles, 72, problems=problems)) == splits
+    # one range asked for: no workspace; two: theirs
+    assert _splits(_attn(rows, 64 * tiles, 72, problems=problems, kv_splits=1)) == 1
+    assert _splits(_attn(rows, 64 * tiles, 72, problems=problems, kv_splits=2)) == 2
