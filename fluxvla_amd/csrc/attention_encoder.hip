@@ -238,7 +238,8 @@ __global__ __launch_bounds__(256) void attn_encoder_kernel(fvx_attn_desc p, int 
 }
 
 // One query head per problem, every key visible, whole key tiles and one key
-// range, head dim <= 80, 8-byte output rows, operand views below 2 GiB; the scale
+// range, head dim <= 80, 8-byte output rows, operand views below 2 GiB, fewer than
+// 2^32 threads (a launch's limit; the general kernel's grid has three axes); the scale
 // is positive, so that the largest score is the largest product, and at most 1 in
 // base 2, so that scaling cannot overflow.
 bool encoder_attn_ok(const fvx_attn_desc& d) {
@@ -251,7 +252,7 @@ bool encoder_attn_ok(const fvx_attn_desc& d) {
          (d.sk + 2 * kEncKT) * d.k_tok_stride < lim &&
          (d.sk + 2 * kEncKT) * d.v_tok_stride < lim && ((uintptr_t)d.o & 7u) == 0 &&
          d.o_tok_stride % 4 == 0 && d.o_zs1 % 4 == 0 && d.o_zs2 % 4 == 0 &&
-         d.n_problems * ((d.sq + 63) / 64) < lim;
+         d.n_problems * ((d.sq + 63) / 64) < ((int64_t)1 << 24);
 }
 
 // 128 rows per workgroup once blocks of 64 number more than the CUs, 64 before.

@@ -78,3 +78,17 @@ def test_few_rows_many_keys(n, sq, sk, hd, ws, splits):
     err = (o[:, :sq].float() - ref).abs().max().item()
     assert err <= 4 * 2.0**-8 * ref.abs().max().item(), err
     assert (o[:, sq:] == 7).all()
+
+
+def test_more_problems_than_one_grid_axis():
+    """2^24 problems of one row, the general kernel's: 2^32 threads of the encoder's."""
+    n, hd = 1 << 24, 8
+    g = torch.Generator(device='cuda').manual_seed(5)
+    q = torch.randn(n, 1, hd, generator=g, device='cuda').to(torch.bfloat16)
+    k, v = torch.randn(2, 64, hd, generator=g, device='cuda').to(torch.bfloat16)
+    o = torch.zeros_like(q)
+    K.mqa_attention(q, k[None].expand(n, -1, -1), v[None].expand(n, -1, -1), o)
+    s = torch.matmul(q[:, 0].float(), k.float().t()) * hd**-0.5
+    ref = torch.matmul(torch.softmax(s, -1), v.float())
+    # bf16 probabilities and output: 2^-8 of the largest value, four of them
+    assert (o[:, 0].float() - ref).abs().max().item() <= 4 * 2.0**-8 * v.abs().max().item()
