@@ -158,6 +158,7 @@ SIGNATURES = {
     'fvx_version': (c_i32, []),
     'fvx_last_error': (ctypes.c_char_p, []),
     'fvx_gemm_workspace_bytes': (c_i64, [ctypes.POINTER(GemmDesc)]),
+    'fvx_gemm_kernel': (ctypes.c_char_p, [ctypes.POINTER(GemmDesc)]),
     'fvx_gemm': (c_i32, [ctypes.POINTER(GemmDesc), c_vp]),
     'fvx_gemm_noalloc': (c_i32, [ctypes.POINTER(GemmDesc), c_vp]),
     'fvx_rms_norm_residual':

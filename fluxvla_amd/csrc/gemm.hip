@@ -2265,6 +2265,22 @@ extern "C" int64_t fvx_gemm_workspace_bytes(const fvx_gemm_desc* d) {
   return need < ((int64_t)1 << 31) ? need : 0;  // larger: the launch runs unsplit
 }
 
+// The kernel that fvx_gemm takes for d (validated), as its tests name it.
+extern "C" const char* fvx_gemm_kernel(const fvx_gemm_desc* d) {
+  if (!d || d->m <= 0) return "none";
+  if (use_skinny(*d)) return "skinny";
+  static const char* const kMid[] = {"mid 64x64", "mid 64x128", "mid 128x128"};
+  const int mid = plan_mid(*d);
+  if (mid >= 0) return kMid[mid];
+  static const char* const kPp[] = {"pp 256x256", "pp 256x320", "pp 256x192", "pp 256x128",
+                                    "pp 128x256"};
+  const int pp = plan_pp(*d);
+  if (pp >= 0) return kPp[pp];
+  const TilePlan t = plan_tile(*d);
+  if (t.cfg == kWideCfg) return t.splits > 1 ? "wide split" : "wide";
+  return t.cfg == kSmallCfg ? "tile 64x64" : (t.cfg == 1 ? "tile 256x256" : "tile 64x128");
+}
+
 // Skinny GEMMs with the adaptive RMSNorm folded in (a_scale): QKV_ROPE,
 // GEGLU and EULER, bf16 or W8A16 weights.
 template <int MODE>

@@ -265,6 +265,10 @@ const char* fvx_last_error(void);
  * one pass).  M <= 64 problems split K in ranges of at most 256; split_k > 0
  * requests a range length of ceil(K / split_k) (still capped at 256). */
 int64_t fvx_gemm_workspace_bytes(const fvx_gemm_desc* d);
+/* The kernel and tile that fvx_gemm takes for the given problem, as a name
+ * ("skinny", "mid 64x128", "pp 256x192", "wide", "tile 64x128", ...): a diagnostic,
+ * of which only the first word's meaning is stable. */
+const char* fvx_gemm_kernel(const fvx_gemm_desc* d);
 
 /* General GEMM with fused epilogue.  Replaces the reference's
  * matmul_bias_cuda (fluxvla/ops/cuda/matmul_bias/matmul_bias.py:19-60,

@@ -1,5 +1,5 @@
 """Which kernel, and how many key ranges, a call takes: the rules of the dispatch as
-its workspace query shows them (no GPU needed; 256 CUs are assumed without one)."""
+its queries show them (no GPU needed; 256 CUs are assumed without one)."""
 import ctypes
 
 import pytest
@@ -49,3 +49,36 @@ def test_unmasked_one_head(rows, problems, tiles, splits):
     # one range asked for: no workspace; two: theirs
     assert _splits(_attn(rows, 64 * tiles, 72, problems=problems, kv_splits=1)) == 1
     assert _splits(_attn(rows, 64 * tiles, 72, problems=problems, kv_splits=2)) == 2
+
+
+def _gemm(m, n, k, mode=_lib.GEMM_PLAIN, fp8=False, **kw):
+    p = 1 << 20
+    d = _lib.GemmDesc()
+    d.a, d.b, d.c, d.m, d.n, d.k, d.lda, d.ldb, d.ldc = p, p, p, m, n, k, k, k, n
+    d.mode = mode
+    if mode == _lib.GEMM_GEGLU:
+        d.b2 = p
+    if mode == _lib.GEMM_QKV_ROPE:
+        d.head_dim, d.n_q_heads = 256, n // 256 - 2
+        d.rope = d.positions = d.q_out = d.k_out = d.v_out = p
+        d.ldq, d.ldk, d.ldv = max(1, d.n_q_heads) * 256, 256, 256
+    if fp8:
+        d.b_fp8, d.b_scale, d.b2_scale = 1, p, p
+    for key, v in kw.items():
+        setattr(d, key, v)
+    return d
+
+
+def _kernel(*args, **kw):
+    return _lib.load().fvx_gemm_kernel(ctypes.byref(_gemm(*args, **kw))).decode()
+
+
+@pytest.mark.parametrize('kernel,args', [
+    ('skinny', (64, 1024, 1024)), ('mid 64x64', (65, 1024, 1024)),
+    ('mid 128x128', (768, 3456, 1152)), ('pp 256x320', (6528, 2560, 2048)),
+    ('tile 64x128', (768, 4308, 1152)), ('wide', (816, 16384, 2048, _lib.GEMM_GEGLU)),
+    ('wide split', (816, 2048, 16384)), ('pp 256x256', (816, 16384, 2048, _lib.GEMM_GEGLU, True)),
+    ('tile 64x128', (408, 4096, 1024, _lib.GEMM_GEGLU, True))])
+def test_gemm_kernel_names(kernel, args):
+    assert _kernel(*args) == kernel
+    assert _lib.load().fvx_gemm_kernel(None) == b'none'
