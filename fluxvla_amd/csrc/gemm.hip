@@ -589,7 +589,8 @@ __global__ __launch_bounds__(64 * NWV, 1) void gemm_wide_kernel(GemmArgs p, int 
   const int lid = xcd_remap(blockIdx.x, nblk * splits);
   const int bid = lid % nblk, split = lid / nblk;
   int m_tile, n_tile;
-  tile_order(bid, m_tiles, n_tiles, kWideRowBlock, m_tile, n_tile);
+  tile_order(bid, m_tiles, n_tiles, splits > 1 ? kWideRowBlock : wide_row_block(m_tiles, p.m),
+             m_tile, n_tile);
   const int64_t M = p.m, N = p.n, K = p.k;
   const int64_t m0 = (int64_t)m_tile * kGwBM, n0 = (int64_t)n_tile * (GG ? 128 : 256);
   // K range [kb, kb + 64 nk) (splits > 1: PLAIN without rownorm, fp32
@@ -897,7 +898,8 @@ __global__ __launch_bounds__(256, 1) void gemm_wide_f8_kernel(GemmArgs p, int m_
   const int lid = xcd_remap(blockIdx.x, nblk * splits);
   const int bid = lid % nblk, split = lid / nblk;
   int m_tile, n_tile;
-  tile_order(bid, m_tiles, n_tiles, kWideRowBlock, m_tile, n_tile);
+  tile_order(bid, m_tiles, n_tiles, splits > 1 ? kWideRowBlock : wide_row_block(m_tiles, p.m),
+             m_tile, n_tile);
   const int64_t M = p.m, N = p.n, K = p.k;
   const int64_t m0 = (int64_t)m_tile * kGwBM, n0 = (int64_t)n_tile * (GG ? 128 : 256);
   // K range [kb, kb + 64 nk) (splits > 1: PLAIN without rownorm, partials

@@ -27,6 +27,16 @@ constexpr int kMaxSkinnyTiles = kCounterBytes / 4;
 constexpr int kTileRowBlock = 16;  // tiles of 64 rows
 constexpr int kWideRowBlock = 4;   // tiles of 256 rows
 
+// The wide kernels skip the rows that a short last tile row lacks, so its tiles are
+// cheap, and in blocks of rows one XCD gets many of them and another none: where more
+// than 1/16 of the tiles' rows are missing, one block of all rows, which spreads them.
+// Gate/up in blocks / one block (us): 1632 x 2 x 16384 x 2048 (9 % missing) 239 / 229,
+// 2086 x 2 x 4096 x 1152 W8A16 (9 %) 88 / 83, 2448 x 2 x 16384 x 2048 (4 %) 316 / 313,
+// 2934 x 2 x 4184 x 1024 (4 %) 64 / 67, 3264 rows (2 %) 430 / 436, 6528 (2 %) 821 / 849.
+__device__ __forceinline__ int wide_row_block(int m_tiles, int64_t M) {
+  return 16 * m_tiles < m_tiles * 256 - (int)M ? m_tiles : kWideRowBlock;
+}
+
 
 // Row indices and the epilogue's periods (row_group, gate_group,
 // pos_period, rtc_period) are below 2^31 (the host checks), so quotients and

@@ -25,3 +25,18 @@ def cuda():
 def announce(msg):
     """Print the case about to run on the GPU, flushed, so a crash names it."""
     print(f'[case] {msg}', flush=True)
+
+
+@pytest.fixture
+def kernels_run(monkeypatch):
+    """The kernels that the test's GEMM calls took, in order (fvx_gemm_kernel)."""
+    from fluxvla_amd import _lib
+    names, call = [], _lib.call
+
+    def recorded(name, *args):
+        if name in ('fvx_gemm', 'fvx_gemm_noalloc'):
+            names.append(_lib.load().fvx_gemm_kernel(args[0]).decode())
+        return call(name, *args)
+
+    monkeypatch.setattr(_lib, 'call', recorded)
+    return names

@@ -50,6 +50,26 @@ def test_geglu_row_blocks(m, fp8):
     _close(got.cpu(), torch.nn.functional.gelu(g, approximate='tanh') * u)
 
 
+# the wide kernel's tile rows in blocks of about 4 (1264, 2300 rows) and, with a short
+# last tile row, in one block (1025, 1632, 2086)
+# (and W8A8: activations that e4m3 holds exactly)
+@pytest.mark.parametrize('fp8', [False, True])
+@pytest.mark.parametrize('m', [1025, 1264, 1632, 2086, 2300])
+def test_wide_row_blocks(m, fp8, kernels_run):
+    n, k = 8200, 128
+    x = torch.randint(-8, 9, (m, k), generator=torch.Generator().manual_seed(6)).to(BF16).cuda()
+    wg, wu = _rand((n, k), 7, 0.01).cuda(), _rand((n, k), 8, 0.01).cuda()
+    if fp8:
+        qg, qu = (K.Fp8Weight.quantize(w, act='e4m3') for w in (wg, wu))
+        got = K.gemm_geglu(x, qg, qu)
+        wg, wu = qg.dequantize(), qu.dequantize()
+    else:
+        got = K.gemm_geglu(x, wg, wu)
+    assert kernels_run == ['wide']
+    g, u = x.float() @ wg.float().t(), x.float() @ wu.float().t()
+    _close(got, torch.nn.functional.gelu(g, approximate='tanh') * u)
+
+
 # gemm_pp_kernel: the sizes at which the plan takes its tiles of 256 x 128, 256 x
 # 192, 256 x 320 and 256 x 256 (the next test: 128 x 256), with rows and columns
 # one past a tile and ragged, and K with a partial last slab (k % 64 != 0); at
