@@ -349,6 +349,12 @@ static bool pp_ok(const GemmArgs& d) {
 // tiles: a second round of four), down 816 rows 221 / 74 (split K) and the
 // expert's gate|up 400 x 2 x 4096 x 1024 29 / 15.  bf16 gate|up stays with the
 // wide kernel, which moves 128 x 128 per wave: 6528 rows 754 / 750, 816 118 / 115.
+// Below 8 slabs the tiles' epilogue, one per CU and not behind another workgroup's K
+// loop, is most of the time, and CUs without a tile are lost to it: at least 176 of 256
+// must have one (us, this / tile kernel: 140 to 169 tiles 5582 x 1280 x 80 15.7 / 14.4, 2609
+// x 2560 x 136 17.1 / 16.1, 1641 x 4096 x 432 21.3 / 19.7, 6961 x 1024 x 272 18.8 / 17.2;
+// 184 to 234 tiles 1978 x 4304 x 136 16.6 / 18.4, 4653 x 2048 x 72 16.7 / 17.9, 5309 x 3456
+// x 416 34.4 / 42.0; but 195 tiles 3801 x 4096 x 112 26.9 / 24.2).
 int plan_pp(const GemmArgs& d) {
   if (!pp_ok(d)) return -1;
   const int cus = device_cus();
@@ -364,6 +370,7 @@ int plan_pp(const GemmArgs& d) {
     // built for 256 x 2 x 128 only
     if ((d.ss_out && (c == 1 || c == 2)) || (gg && c) || (d.b_fp8 && t.slab8 == 0.f)) continue;
     const int64_t tiles = ((d.m + t.bm - 1) / t.bm) * ((d.n * nb + t.bn - 1) / t.bn);
+    if (slabs < 8.f && 16 * tiles < 11 * cus) continue;
     const float us = (float)((tiles + cus - 1) / cus) *
                      (d.b_fp8 ? slabs * t.slab8 + t.fixed8 : slabs * t.slab + t.fixed);
     if (us < best) {

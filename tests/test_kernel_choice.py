@@ -82,3 +82,13 @@ def _kernel(*args, **kw):
 def test_gemm_kernel_names(kernel, args):
     assert _kernel(*args) == kernel
     assert _lib.load().fvx_gemm_kernel(None) == b'none'
+
+
+# few slabs: the two-group kernel from 176 tiles on (256 CUs)
+@pytest.mark.parametrize('m,n,k,pp', [(1641, 4096, 432, False), (5582, 1280, 80, False),
+                                      (6961, 1024, 272, False), (5309, 3456, 416, True),
+                                      (1978, 4304, 136, True), (14235, 3456, 144, True),
+                                      (1804, 3456, 1024, True)])
+def test_two_group_kernel_at_short_k(m, n, k, pp):
+    assert _kernel(m, n, k).startswith('pp') == pp
+    assert not _kernel(m, n + 4, k).startswith('pp')  # (columns in eights)
