@@ -1069,27 +1069,6 @@ constexpr int64_t kDtTargetWgs = 256;
 // MFMA steps ahead of their use (deeper rings measured no faster)
 constexpr int kDtAhead = 6, kDtRing = kDtAhead + 2;
 
-// The values of lanes l and l ^ 32 combined in both (v_permlane32_swap: a
-// VALU exchange of the wave's halves, where a shuffle is an LDS round trip).
-// Both lanes compute the same expression of the same two values, so they
-// agree bit for bit.
-__device__ __forceinline__ void half_pair(float v, float& a, float& b) {
-  const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v),
-                                                  false, false);
-  a = __uint_as_float(s[0]);  // lane l & 31's value
-  b = __uint_as_float(s[1]);  // lane (l & 31) + 32's value
-}
-__device__ __forceinline__ float half_pair_max(float v) {
-  float a, b;
-  half_pair(v, a, b);
-  return fmaxf(a, b);
-}
-__device__ __forceinline__ float half_pair_sum(float v) {
-  float a, b;
-  half_pair(v, a, b);
-  return a + b;
-}
-
 // NW = 2 or 4 waves: with 4, every K / V^T tile brought into the LDS serves
 // 128 query rows and all four SIMDs of the CU.  n_rg counts 64-row groups
 // (the unit of the partials and of the merge); a 4-wave workgroup covers two

@@ -29,15 +29,9 @@ constexpr int kEncLDK = 96 + 8, kEncLDV = 64 + 8;  // LDS row lengths (elements)
 constexpr int kEncND = 5, kEncNS = 3;             // 16-dim blocks of O, 32-dim steps of QK^T
 constexpr int kEncK = kEncKT * kEncLDK, kEncV = 16 * kEncND * kEncLDV;
 
-// the values of lanes l and l ^ 16, or l and l ^ 32
+// the values of lanes l and l ^ 16 (half_pair: l and l ^ 32)
 __device__ __forceinline__ void enc_pair16(float v, float& a, float& b) {
   const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false,
-                                                  false);
-  a = __uint_as_float(s[0]);
-  b = __uint_as_float(s[1]);
-}
-__device__ __forceinline__ void enc_pair32(float v, float& a, float& b) {
-  const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false,
                                                   false);
   a = __uint_as_float(s[0]);
   b = __uint_as_float(s[1]);
@@ -177,8 +171,7 @@ __global__ __launch_bounds__(256) void attn_encoder_kernel(fvx_attn_desc p, int 
         for (int e = 0; e < 4; ++e) mx = fmaxf(mx, s[r][kf][e]);
       enc_pair16(mx, a, b);
       mx = fmaxf(a, b);
-      enc_pair32(mx, a, b);
-      mx = fmaxf(a, b);
+      mx = half_pair_max(mx);
       const float m_new = fmaxf(m_run[r], mx * sc);
       const float m_ref = m_new == -INFINITY ? 0.f : m_new;
       const float alpha = __builtin_amdgcn_exp2f(m_run[r] - m_ref);
@@ -223,8 +216,7 @@ __global__ __launch_bounds__(256) void attn_encoder_kernel(fvx_attn_desc p, int 
   for (int r = 0; r < RG; ++r) {
     float a, b;
     enc_pair16(l_run[r], a, b);
-    enc_pair32(a + b, a, b);
-    const float l = a + b, inv = l > 0.f ? 1.f / l : 0.f;
+    const float l = half_pair_sum(a + b), inv = l > 0.f ? 1.f / l : 0.f;
     const int row = rb * (64 * RG) + (wave * RG + r) * 16 + fr;
     if (row < sq) {
       bf16_t* orow = O + (int64_t)row * p.o_tok_stride + 4 * g;

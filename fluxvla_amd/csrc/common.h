@@ -213,6 +213,27 @@ __device__ __forceinline__ i32x4_t make_rsrc4(const void* base, uint32_t bytes) 
   return r;
 }
 
+// The values of lanes l and l ^ 32 combined in both (v_permlane32_swap: a
+// VALU exchange of the wave's halves, where a shuffle is an LDS round trip).
+// Both lanes compute the same expression of the same two values, so they
+// agree bit for bit.
+__device__ __forceinline__ void half_pair(float v, float& a, float& b) {
+  const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v),
+                                                  false, false);
+  a = __uint_as_float(s[0]);  // lane l & 31's value
+  b = __uint_as_float(s[1]);  // lane (l & 31) + 32's value
+}
+__device__ __forceinline__ float half_pair_max(float v) {
+  float a, b;
+  half_pair(v, a, b);
+  return fmaxf(a, b);
+}
+__device__ __forceinline__ float half_pair_sum(float v) {
+  float a, b;
+  half_pair(v, a, b);
+  return a + b;
+}
+
 // Workgroups are dispatched round-robin over the 8 XCDs (workgroup b of a
 // 1-D grid runs on XCD b % 8), and each XCD has its own L2.  xcd_remap gives
 // XCD x the contiguous logical ids [start(x), start(x) + count(x)), count(x)

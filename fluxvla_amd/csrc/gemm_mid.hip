@@ -20,13 +20,6 @@
 
 namespace fvx {
 
-// the sum of lanes l and l ^ 32, in both
-__device__ __forceinline__ float mid_half_sum(float v) {
-  const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false,
-                                                  false);
-  return __uint_as_float(s[0]) + __uint_as_float(s[1]);
-}
-
 template <int RB, int JN, int WGM, int WGN, int KG, int NST>
 struct MidCfg {
   static constexpr int BM = 32 * RB * WGM, BN = 32 * JN * WGN;
@@ -202,9 +195,9 @@ __global__ __launch_bounds__(512, 1) void gemm_mid_kernel(GemmArgs p, int m_tile
         a += prt[i][q];
       }
       for (int q = PR; 2 * q < p.ss_parts; ++q) a += part(i, q);
-      rf[i] = rsqrtf(mid_half_sum(a) / (float)K + p.rownorm_eps);
+      rf[i] = rsqrtf(half_pair_sum(a) / (float)K + p.rownorm_eps);
     }
-    if constexpr (SUMX) ss[i] = mid_half_sum(ss[i]);
+    if constexpr (SUMX) ss[i] = half_pair_sum(ss[i]);
   }
   if (AC == 2)
 #pragma unroll
@@ -305,7 +298,7 @@ __global__ __launch_bounds__(512, 1) void gemm_mid_kernel(GemmArgs p, int m_tile
     if constexpr (HOX) {
       // the row's sum over the wave's 64 columns (JN = 2), over both groups
       static_assert(!HOX || (JN == 2 && RB == 1), "one 64-column block per wave");
-      q = mid_half_sum(q);
+      q = half_pair_sum(q);
       if (KG == 2) {
         hand_ex[(kg * NW + w) * 32 + fr] = q;
         __syncthreads();
@@ -340,9 +333,9 @@ static bool mid_ok(const GemmArgs& d) {
 //      1024 12.6 -> 9.6.  Not for the plain one: 1536 x 1152 x 1152 10.1 -> 10.4,
 //      1632 x 1024 x 4096 21.4 -> 23.0.
 //   0: 64 x 64, two K groups: expert O 408 x 1024 x 2048 9.6 -> 8.4, down 408 x
-//      1024 x 4096 15.2 -> 14.1, SigLIP o 768 x 1152 x 1152 7.4 -> 7.2; fc2 (K =
-//      4304, 22.9 -> 22.6) is bound by its loads, whose 128-byte rows straddle two
-//      cache lines.
+//      1024 x 4096 15.2 -> 14.1, SigLIP o 768 x 1152 x 1152 7.4 -> 7.2, fc2 768 x
+//      1152 x 4304 22.9 -> 22.6 (68.7 MB fetched for 16.5 MB of operands: an XCD's
+//      27 tiles cover all 12 tile rows, so all of A passes through each of 8 L2s).
 // From K = 8192 on the wide kernel's K ranges are faster (prefix down 816 x 2048 x
 // 16384: 78 us against about 84).
 int plan_mid(const GemmArgs& d) {

@@ -29,13 +29,6 @@ __device__ __forceinline__ void pp_bar() {
   asm volatile("" ::: "memory");
 }
 
-// the sum of lanes l and l ^ 32, in both
-__device__ __forceinline__ float pp_half_sum(float v) {
-  const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false,
-                                                  false);
-  return __uint_as_float(s[0]) + __uint_as_float(s[1]);
-}
-
 template <int RB, int JN, int WGM, int WGN, int NST, bool F8>
 struct PpCfg {
   static constexpr int BM = 32 * RB * WGM, BN = 32 * JN * WGN;
@@ -155,7 +148,7 @@ __global__ __launch_bounds__(512, 1) void gemm_pp_kernel(GemmArgs p, int m_tiles
 #pragma unroll
         for (int u = 0; u < 16; ++u) a += v[u];
       }
-      rf[i] = rsqrtf(pp_half_sum(a) / (float)K + p.rownorm_eps);
+      rf[i] = rsqrtf(half_pair_sum(a) / (float)K + p.rownorm_eps);
     }
   }
 
@@ -237,7 +230,7 @@ __global__ __launch_bounds__(512, 1) void gemm_pp_kernel(GemmArgs p, int m_tiles
   wait_vmcnt<0>();
   if constexpr (SUMX) {
 #pragma unroll
-    for (int i = 0; i < RB; ++i) rf[i] = rsqrtf(pp_half_sum(ss[i]) / (float)K + p.rownorm_eps);
+    for (int i = 0; i < RB; ++i) rf[i] = rsqrtf(half_pair_sum(ss[i]) / (float)K + p.rownorm_eps);
   }
 
   // Epilogue: block (i, j) of lane (fr, hk) holds row 32 i + fr, columns 8 (r
@@ -297,7 +290,7 @@ __global__ __launch_bounds__(512, 1) void gemm_pp_kernel(GemmArgs p, int m_tiles
       if constexpr (HOX) {
         // the row's sum over a 64-column block (two 32-column blocks)
         if (j & 1) {
-          const float t = pp_half_sum(q);
+          const float t = half_pair_sum(q);
           const int blk = (n0 + 32 * (JN * wn + j - 1)) >> 6;
           if (hk == 0 && m < M && 64 * blk < N) p.ss_out[(int64_t)blk * p.ss_ld + m] = t;
           q = 0.f;
