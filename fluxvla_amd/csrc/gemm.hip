@@ -4,18 +4,23 @@
 //
 // Kernels (all share the 8-column epilogue epi_load / epi_store):
 //
-//  * gemm_tile_kernel<BM, BN, WGM, WGN, STAGES, MODE, FP8>: M > 64 (SigLIP
-//    M=768, Gemma prefix M=816, batched expert).  64 x 128 tiles of 2 x 2
+//  * gemm_mid_kernel (gemm_mid.hip): M > 64, bf16 PLAIN, GEGLU and Q|K|V GEMMs of
+//    one round of small tiles (SigLIP M=768 and prefix M=816 but its gate/up and
+//    down, the batched expert).
+//  * gemm_pp_kernel (gemm_pp.hip): PLAIN and Q|K|V GEMMs with enough rows for its
+//    larger tiles to fill the CUs (batched SigLIP and prefix), with e4m3 weights
+//    and bf16 activations GEGLU too.
+//  * gemm_tile_kernel<BM, BN, WGM, WGN, STAGES, MODE, FP8>: M > 64, what neither
+//    serves (the W8A16 expert's batches, W8A8, EULER, a folded LayerNorm, N not
+//    a multiple of 8, sizes between the two).  64 x 128 tiles of 2 x 2
 //    waves on v_mfma_f32_32x32x16_bf16 (fp8: the block-scaled 32x32x64), K in
 //    64-wide slabs through a 3- or 4-stage LDS ring filled by LDS DMA
 //    (buffer_load ... lds), the slab loads spread between MFMA groups.
 //  * gemm_wide_kernel<MODE, SUM_A, NWV> / gemm_wide_f8_kernel: 256 x 256
 //    tiles of 8 waves (64 x 128 each; fp8: 4 waves of 128 x 128, the
-//    accumulators in AGPRs) for the prefix gate/up
-//    at every batch, batched prefixes, and -- over up to 8 K ranges, one
-//    per XCD -- long-K GEMMs with few tiles (the prefix down projection).
-//  * gemm_pp_kernel (gemm_pp.hip): bf16 PLAIN and Q|K|V GEMMs with enough
-//    rows for its larger tiles to fill the CUs (batched SigLIP and prefix).
+//    accumulators in AGPRs) for the bf16 prefix gate/up at every batch, W8A8
+//    prefixes, and -- over up to 8 K ranges, one per XCD -- long-K GEMMs with
+//    few tiles (the prefix down projection).
 //  * gemm_skinny_kernel<MODE, FP8>: M <= 64 (the bs=1 action expert,
 //    M=50/51).  A weight stream: a workgroup owns 16 output columns and
 //    reads its weight rows straight from memory as MFMA B fragments
@@ -24,8 +29,9 @@
 //  * gemm_partial_reduce_kernel: the split-K sum (in split order,
 //    deterministic) and epilogue behind the tile and wide kernels.
 //
-// Tiles are ordered m-fastest within blocks of about 1024 rows (tile_order)
-// and block ids remapped (xcd_remap) so that one XCD owns consecutive tiles:
+// Tiles are ordered m-fastest within blocks of rows (tile_order; one-round
+// kernel: within all rows) and block ids remapped (xcd_remap) so that one XCD
+// owns consecutive tiles:
 // the tiles of a block run on one XCD and reuse its rows of A and its weight
 // panels from the L2.
 //
@@ -1935,7 +1941,9 @@ static int validate(const GemmArgs& d) {
 //      of 8 waves per CU; half the L2 traffic per flop of a 128 x 128 tile)
 //   2:  64 x 128 with 4 stages (96 KiB, one workgroup per CU: three slabs in
 //       flight instead of one, for grids that leave CUs free anyway)
-// Measured on MI355X (us; bs=1 chunk shapes):
+// Measured on MI355X (us; bs=1 chunk shapes, of which the bf16 ones with whole
+// chunks of 8 columns have since gone to the one-round kernel; the rule is for
+// what that leaves):
 //   prefix GeGLU 816 x 16384 x2 x 2048   128x128: 158, 1: 151 (0: 154)
 //   prefix QKV   816 x 2560 x 2048   (260 tiles)   0: 26.2   2: 37.4
 //   prefix O     816 x 2048 x 2048   (208 tiles)   0: 23.7   2: 19.9
@@ -1950,8 +1958,8 @@ static const int kTileBN[] = {128, 256, 128, 256, 64};
 constexpr int kTileCfgs = 5;
 constexpr int kWideCfg = 3;  // gemm_wide_kernel
 // 4: 64 x 64, 2 x 2 waves of 32 x 32, 4 stages -- bf16 PLAIN / QKV / EULER
-// GEMMs with fewer than 128 tiles of 64 x 128 (SigLIP o-proj, fc2: M = 768,
-// N = 1152): twice the workgroups instead of idle CUs or a split-K pass
+// GEMMs with fewer than 128 tiles of 64 x 128 that the one-round kernel does
+// not serve: twice the workgroups instead of idle CUs or a split-K pass
 constexpr int kSmallCfg = 4;
 #ifndef FVX_WIDE_MIN_TILES
 #define FVX_WIDE_MIN_TILES 128

@@ -18,14 +18,15 @@ constexpr int64_t kEpiRows = 256;
 constexpr int kCounterBytes = 4096;
 constexpr int kMaxSkinnyTiles = kCounterBytes / 4;
 
-// Tile rows per block of the tile order (tile_order): about 1024 rows.  One
+// Tile rows per block of the tile order (tile_order): about 1024 rows of the 64 x 128
+// and wide tiles (the tile kernel's 128- and 256-row tiles: 2048 and 4096).  One
 // block of all rows against this, us (MI355X, weights from HBM): prefix down
 // 6528 x 2048 x 16384 538 -> 428 (all 26 tile rows on every XCD streamed A
 // eight times), gate/up 6528 x 2 x 16384 x 2048 775 -> 750, Q|K|V 107 -> 98;
 // SigLIP fc1 6144 x 4304 x 1152 97 -> 89, Q|K|V 81 -> 75, fc2 120 -> 114; fp8
 // gate/up at 22144 rows 2970 -> 2850.  Blocks of 2048 rows: gate/up 785.
-constexpr int kTileRowBlock = 16;  // tiles of 64 rows
-constexpr int kWideRowBlock = 4;   // tiles of 256 rows
+constexpr int kTileRowBlock = 16;  // of the tile kernel
+constexpr int kWideRowBlock = 4;   // of 256 rows
 
 // The wide kernels skip the rows that a short last tile row lacks, so its tiles are
 // cheap, and in blocks of rows one XCD gets many of them and another none: where more

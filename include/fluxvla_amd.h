@@ -155,7 +155,7 @@ typedef struct fvx_gemm_desc {
    *           64-column block of n of bf16(c[m][n'])^2 (ceil(N / 64) parts);
    *   ss_in  (rownorm): the sum of squares of row m of A is taken as
    *           ss_in[0 * ss_ld + m] + ... + ss_in[(ss_parts - 1) * ss_ld + m],
-   *           added in that order (deterministic). */
+   *           added in a fixed order of the kernel's own (deterministic). */
   float* ss_out;
   const float* ss_in;
   int64_t ss_ld;
@@ -242,8 +242,8 @@ typedef struct fvx_gemm_desc {
    * the same two values): gu_out (may be NULL) receives per output row the
    * bf16 gate values (columns n) and up values (columns N + n) that the
    * product gelu_tanh(gate) * up is taken from, row stride ld_gu >= 2 N.
-   * GEGLU mode on the skinny and tile kernels (the wide kernel is not used
-   * with it). */
+   * GEGLU mode on the skinny and tile kernels (no other kernel is used with
+   * it). */
   void* gu_out;
   int64_t ld_gu;
   /* QKV_ROPE with v_transposed, copies in the other layouts (no
