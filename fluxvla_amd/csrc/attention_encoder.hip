@@ -247,17 +247,19 @@ bool encoder_attn_ok(const fvx_attn_desc& d) {
          d.n_problems * ((d.sq + 63) / 64) < ((int64_t)1 << 24);
 }
 
-// 128 rows per workgroup once blocks of 64 number more than the CUs, 64 before.
+// 128 rows per workgroup once blocks of 64 number more than the CUs and two of them
+// share a problem, 64 else.
 // Measured (us per call, images of 256 patches, 16 heads of 72: attn_kernel / 64
 // rows / 128 rows): 1 image 11.7 / 7.2 / 9.3, 3 images 13.9 / 7.4 / 9.5, 5 images
 // 18.0 / 9.9 / 9.8, 24 images 44.8 / 27.1 / 23.4, 96 images 148 / 90 / 74 (390
-// TFLOP/s).  Two groups of 4 waves with every other tile each were no faster at 1 to
+// TFLOP/s).  4000 problems of 64 rows x 512 keys 164 / 140 / 170: half of 128 rows are
+// absent there.  Two groups of 4 waves with every other tile each were no faster at 1 to
 // 3 images (7.4 to 7.7).
 int run_encoder_attn(const fvx_attn_desc& d, hipStream_t s) {
   const uint32_t kch = (uint32_t)(d.head_dim / 8);
   const uint32_t magic = (65536u + kch - 1) / kch;  // i / kch for i < 768
   const int64_t n64 = (d.sq + 63) / 64, n128 = (d.sq + 127) / 128;
-  if (d.n_problems * n64 <= device_cus())
+  if (d.n_problems * n64 <= device_cus() || n64 == n128)
     hipLaunchKernelGGL((attn_encoder_kernel<1>), dim3((unsigned)(d.n_problems * n64)), dim3(256),
                        0, s, d, (int)n64, magic);
   else

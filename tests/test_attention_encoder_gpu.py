@@ -9,12 +9,12 @@ from fluxvla_amd import kernels as K
 pytestmark = pytest.mark.gpu
 
 
-# 64 rows per workgroup up to 256 blocks of 64 rows (one per CU), then 128; one, an
-# odd and an even number of key tiles, ragged rows
+# 64 rows per workgroup up to 256 blocks of 64 rows (one per CU) and for problems of up to
+# 64 rows, else 128; one, an odd and an even number of key tiles, ragged rows
 @pytest.mark.parametrize('n,sq,sk,hd', [
     (1, 1, 64, 8), (3, 65, 128, 72), (2, 200, 192, 80), (48, 256, 256, 72),
     (100, 130, 64, 40), (90, 257, 320, 72), (200, 130, 192, 80), (384, 256, 256, 72),
-    (256, 64, 64, 72), (257, 1, 64, 72),
+    (256, 64, 64, 72), (257, 1, 64, 72), (257, 64, 192, 72), (257, 65, 192, 72),
     # the general kernel: keys past the last whole tile
     (3, 100, 100, 72)])
 def test_unmasked(n, sq, sk, hd):
