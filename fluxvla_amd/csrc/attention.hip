@@ -1550,7 +1550,7 @@ static AttnPlan plan_attn_fitting(const fvx_attn_desc& d) {
 // attn_encoder_kernel where it can serve d, or attn_kernel over the plan's key
 // ranges and the merge: the encoder kernel walks all T key tiles in one workgroup
 // and takes about 2.8 + 0.93 T us while 64-row blocks have a CU each, attn_kernel
-// with ranges of t tiles and its merge 6.1 to 7.4 + 2.1 t with 1 to 32 blocks (and more
+// with ranges of t tiles and its merge 6.1 to 8 + 2.1 t with 1 to 48 blocks (and more
 // past them).
 // Measured (us, encoder / general; head dim 72, blocks of 64 rows x tiles): 1 x 8
 // 10.1 / 10.1, 1 x 16 17.7 / 10.4, 1 x 64 61.9 / 17.3; 16 x 8 10.3 / 10.8, 16 x 12
@@ -1559,7 +1559,7 @@ static AttnPlan plan_attn_fitting(const fvx_attn_desc& d) {
 static bool encoder_first(const fvx_attn_desc& d, const AttnPlan& a) {
   const int64_t tiles = d.sk / kKeyTile, range = a.kps / kKeyTile;
   const int64_t blocks = (int64_t)a.n_row_blocks * d.n_problems;
-  return encoder_attn_ok(d) && 4 * tiles <= 14 + (blocks < 32 ? blocks : 32) / 8 + 9 * range;
+  return encoder_attn_ok(d) && 4 * tiles <= 14 + (blocks < 48 ? blocks : 48) / 8 + 9 * range;
 }
 
 extern "C" int64_t fvx_attention_workspace_bytes(const fvx_attn_desc* d) {

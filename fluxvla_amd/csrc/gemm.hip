@@ -576,7 +576,8 @@ constexpr int wide_lds_bytes() {
 template <int MODE, bool SUM_A, int NWV>  // SUM_A: the fused RMSNorm sums A's squares here
 __global__ __launch_bounds__(64 * NWV, 1) void gemm_wide_kernel(GemmArgs p, int m_tiles,
                                                                 int n_tiles, int vec_ok,
-                                                                int splits, int kchunk) {
+                                                                int splits, int kchunk,
+                                                                int row_block) {
   constexpr bool GG = MODE == FVX_GEMM_GEGLU;
   constexpr int WNO = GG ? 64 : 128;  // output columns per wave
   constexpr int WM = NWV == 8 ? 64 : 128, RB = WM / 32;  // rows, row blocks per wave
@@ -595,8 +596,7 @@ __global__ __launch_bounds__(64 * NWV, 1) void gemm_wide_kernel(GemmArgs p, int 
   const int lid = xcd_remap(blockIdx.x, nblk * splits);
   const int bid = lid % nblk, split = lid / nblk;
   int m_tile, n_tile;
-  tile_order(bid, m_tiles, n_tiles, splits > 1 ? kWideRowBlock : wide_row_block(m_tiles, p.m),
-             m_tile, n_tile);
+  tile_order(bid, m_tiles, n_tiles, row_block, m_tile, n_tile);
   const int64_t M = p.m, N = p.n, K = p.k;
   const int64_t m0 = (int64_t)m_tile * kGwBM, n0 = (int64_t)n_tile * (GG ? 128 : 256);
   // K range [kb, kb + 64 nk) (splits > 1: PLAIN without rownorm, fp32
@@ -885,7 +885,8 @@ struct Gw8Layout {
 template <int MODE, bool SUM_A, bool F8A, bool A16>
 __global__ __launch_bounds__(256, 1) void gemm_wide_f8_kernel(GemmArgs p, int m_tiles,
                                                               int n_tiles, int vec_ok,
-                                                              int splits, int kchunk) {
+                                                              int splits, int kchunk,
+                                                              int row_block) {
   static_assert(!(A16 && F8A), "W8A16 reads a bf16 A");
   typedef Gw8Layout<F8A> LY;
   constexpr bool GG = MODE == FVX_GEMM_GEGLU;
@@ -904,8 +905,7 @@ __global__ __launch_bounds__(256, 1) void gemm_wide_f8_kernel(GemmArgs p, int m_
   const int lid = xcd_remap(blockIdx.x, nblk * splits);
   const int bid = lid % nblk, split = lid / nblk;
   int m_tile, n_tile;
-  tile_order(bid, m_tiles, n_tiles, splits > 1 ? kWideRowBlock : wide_row_block(m_tiles, p.m),
-             m_tile, n_tile);
+  tile_order(bid, m_tiles, n_tiles, row_block, m_tile, n_tile);
   const int64_t M = p.m, N = p.n, K = p.k;
   const int64_t m0 = (int64_t)m_tile * kGwBM, n0 = (int64_t)n_tile * (GG ? 128 : 256);
   // K range [kb, kb + 64 nk) (splits > 1: PLAIN without rownorm, partials
@@ -2115,6 +2115,18 @@ static void launch_small_tile(dim3 grid, hipStream_t s, const GemmArgs& d, int x
         grid, s, d, xf, m_tiles, n_tiles, splits, kchunk, vec_ok);
 }
 
+// Tile rows per block of the wide kernels' tile order (tile_order): kWideRowBlock, but
+// all in one block where a short last tile row lacks more than 1/16 of the tiles' rows
+// (no K ranges).  The kernels skip those rows, so that row's tiles are cheap, and in
+// blocks one XCD gets many of them and another none.  Gate/up in blocks / one block (us):
+// 1632 x 2 x 16384 x 2048 (9 % missing) 239 / 229, 2086 x 2 x 4096 x 1152 W8A16 (9 %) 88 /
+// 83, 2448 x 2 x 16384 x 2048 (4 %) 316 / 313, 2934 x 2 x 4184 x 1024 (4 %) 64 / 67, 3264
+// rows (2 %) 430 / 436, 6528 (2 %) 821 / 849.
+static int wide_row_block(const GemmArgs& d, int m_tiles, int splits) {
+  const bool blocks = splits > 1 || 16 * m_tiles >= (int64_t)m_tiles * kGwBM - d.m;
+  return blocks ? kWideRowBlock : m_tiles;
+}
+
 static int run_tile(GemmArgs d, int cfg, int splits, hipStream_t s) {
   FVX_REQUIRE(cfg >= 0 && cfg < kTileCfgs, FVX_ERR_ARG, "gemm: bad tile config %d", cfg);
   FVX_REQUIRE(cfg != 1 || d.mode == FVX_GEMM_GEGLU || d.b_fp8, FVX_ERR_ARG,
@@ -2162,35 +2174,36 @@ static int run_tile(GemmArgs d, int cfg, int splits, hipStream_t s) {
     // splits, (split, tile) workgroups
     const unsigned nb = (unsigned)(m_tiles * n_tiles);
     const unsigned nbs = nb * (unsigned)splits;
+    const int rows = wide_row_block(d, m_tiles, splits);
 #define LW(MODE)                                                                       \
   if (d.rownorm && !d.ss_in)                                                           \
     hipLaunchKernelGGL((gemm_wide_kernel<MODE, true, wide_waves<MODE>()>), dim3(nbs),    \
                        dim3(64 * wide_waves<MODE>()), 0, s, d, m_tiles, n_tiles, vec_ok, \
                        splits,                                                         \
-                       (int)kchunk);                                                   \
+                       (int)kchunk, rows);                                             \
   else                                                                                 \
     hipLaunchKernelGGL((gemm_wide_kernel<MODE, false, wide_waves<MODE>()>), dim3(nbs),   \
                        dim3(64 * wide_waves<MODE>()), 0, s, d, m_tiles, n_tiles, vec_ok, \
                        splits,                                                         \
-                       (int)kchunk)
+                       (int)kchunk, rows)
     // the e4m3 copy of A is used when given (a rownorm then needs ss_in)
     const bool f8a = d.a8 && d.a8_scale && (!d.rownorm || d.ss_in);
 #define LW8(MODE)                                                                           \
   if (!d.fp8_act && d.rownorm && !d.ss_in)                                                  \
     hipLaunchKernelGGL((gemm_wide_f8_kernel<MODE, true, false, true>), dim3(nbs), dim3(256), \
-                       0, s, d, m_tiles, n_tiles, vec_ok, splits, (int)kchunk);             \
+                       0, s, d, m_tiles, n_tiles, vec_ok, splits, (int)kchunk, rows);       \
   else if (!d.fp8_act)                                                                      \
     hipLaunchKernelGGL((gemm_wide_f8_kernel<MODE, false, false, true>), dim3(nbs), dim3(256),\
-                       0, s, d, m_tiles, n_tiles, vec_ok, splits, (int)kchunk);             \
+                       0, s, d, m_tiles, n_tiles, vec_ok, splits, (int)kchunk, rows);       \
   else if (d.rownorm && !d.ss_in)                                                           \
     hipLaunchKernelGGL((gemm_wide_f8_kernel<MODE, true, false, false>), dim3(nbs), dim3(256),\
-                       0, s, d, m_tiles, n_tiles, vec_ok, splits, (int)kchunk);             \
+                       0, s, d, m_tiles, n_tiles, vec_ok, splits, (int)kchunk, rows);       \
   else if (f8a)                                                                             \
     hipLaunchKernelGGL((gemm_wide_f8_kernel<MODE, false, true, false>), dim3(nbs), dim3(256),\
-                       0, s, d, m_tiles, n_tiles, vec_ok, splits, (int)kchunk);             \
+                       0, s, d, m_tiles, n_tiles, vec_ok, splits, (int)kchunk, rows);       \
   else                                                                                      \
     hipLaunchKernelGGL((gemm_wide_f8_kernel<MODE, false, false, false>), dim3(nbs),         \
-                       dim3(256), 0, s, d, m_tiles, n_tiles, vec_ok, splits, (int)kchunk)
+                       dim3(256), 0, s, d, m_tiles, n_tiles, vec_ok, splits, (int)kchunk, rows)
     if (d.b_fp8) {
       switch (d.mode) {
         case FVX_GEMM_GEGLU: LW8(FVX_GEMM_GEGLU); break;

@@ -28,17 +28,6 @@ constexpr int kMaxSkinnyTiles = kCounterBytes / 4;
 constexpr int kTileRowBlock = 16;  // of the tile kernel
 constexpr int kWideRowBlock = 4;   // of 256 rows
 
-// The wide kernels skip the rows that a short last tile row lacks, so its tiles are
-// cheap, and in blocks of rows one XCD gets many of them and another none: where more
-// than 1/16 of the tiles' rows are missing, one block of all rows, which spreads them.
-// Gate/up in blocks / one block (us): 1632 x 2 x 16384 x 2048 (9 % missing) 239 / 229,
-// 2086 x 2 x 4096 x 1152 W8A16 (9 %) 88 / 83, 2448 x 2 x 16384 x 2048 (4 %) 316 / 313,
-// 2934 x 2 x 4184 x 1024 (4 %) 64 / 67, 3264 rows (2 %) 430 / 436, 6528 (2 %) 821 / 849.
-__device__ __forceinline__ int wide_row_block(int m_tiles, int64_t M) {
-  return 16 * m_tiles < m_tiles * 256 - (int)M ? m_tiles : kWideRowBlock;
-}
-
-
 // Row indices and the epilogue's periods (row_group, gate_group,
 // pos_period, rtc_period) are below 2^31 (the host checks), so quotients and
 // remainders take the 32-bit unsigned divide: the 64-bit one is a long
@@ -168,8 +157,8 @@ __device__ __forceinline__ void bl_f8(__amdgpu_buffer_rsrc_t r, uint32_t off,
 // output and gate rows) and cover up to kEpiRows rows from there: operands of
 // any size are read right while those rows span less than 2 GiB (validate).
 struct EpiViews {
-  int64_t m0, orow0, grow0;
-  __amdgpu_buffer_rsrc_t bias, bf32, bf32l, gate, res, pos, xt, prev, cw, rope, positions, csum;
+  uint32_t m0, orow0, grow0;  // (offsets from them are taken modulo 2^32)
+  __amdgpu_buffer_rsrc_t bias, bf32, gate, res, pos, xt, prev, cw, rope, positions, csum;
 };
 
 // (SP: the plain-epilogue build -- PLAIN with bias, fp32 bias, activation,
@@ -179,8 +168,8 @@ template <int MODE, bool SP = false>
 __device__ __forceinline__ EpiViews epi_views(const GemmArgs& p, int64_t m0) {
   EpiViews V;
   const int64_t N = p.n, ml = p.m - m0;
-  V.m0 = V.orow0 = V.grow0 = m0;
-  V.bias = V.bf32 = V.bf32l = V.gate = V.res = V.pos = V.xt = V.prev = V.cw = V.rope = V.positions =
+  V.m0 = V.orow0 = V.grow0 = (uint32_t)m0;
+  V.bias = V.bf32 = V.gate = V.res = V.pos = V.xt = V.prev = V.cw = V.rope = V.positions =
       V.csum = make_rsrc(nullptr, 0u);
   if constexpr (SP) {
     V.bias = make_rsrc(p.bias, p.bias ? rec_bytes(N * 2) : 0u);
@@ -198,7 +187,6 @@ __device__ __forceinline__ EpiViews epi_views(const GemmArgs& p, int64_t m0) {
   if (MODE == FVX_GEMM_PLAIN || MODE == FVX_GEMM_EULER) {
     V.bias = make_rsrc(p.bias, p.bias ? rec_bytes(N * 2) : 0u);
     V.bf32 = make_rsrc(p.bias_f32, p.bias_f32 ? rec_bytes(N * 4) : 0u);
-    V.bf32l = make_rsrc(p.bias_f32_locked, p.bias_f32_locked ? rec_bytes(N * 4) : 0u);
   }
   if (MODE == FVX_GEMM_EULER) {
     V.xt = make_rsrc(p.xt + m0 * p.ldx, rec_bytes(ml * p.ldx * 4));
@@ -210,14 +198,15 @@ __device__ __forceinline__ EpiViews epi_views(const GemmArgs& p, int64_t m0) {
     V.csum = make_rsrc(p.ln_csum, p.ln_csum ? rec_bytes(N * 4) : 0u);
     const bool gdiv = p.gate_group > 1;
     const int64_t grows = gdiv ? udiv32(p.m + p.gate_group - 1, p.gate_group) : p.m;
-    V.grow0 = gdiv ? udiv32(m0, p.gate_group) : m0;
+    if (gdiv) V.grow0 = udiv32(m0, p.gate_group);
     V.gate = make_rsrc((const bf16_t*)p.gate + V.grow0 * p.ldg,
                        p.gate ? rec_bytes((grows - V.grow0) * p.ldg * 2) : 0u);
     // (from the start of m0's group: no row of the tile lies before it)
-    if (p.row_group > 0) V.orow0 = (int64_t)udiv32(m0, p.row_group) * p.row_group_stride;
-    V.res = make_rsrc((const bf16_t*)p.residual + V.orow0 * p.ldr,
-                      p.residual ? rec_bytes((out_row(p, p.m - 1) + 1 - V.orow0) * p.ldr * 2)
-                                 : 0u);
+    const int64_t orow0 =
+        p.row_group > 0 ? (int64_t)udiv32(m0, p.row_group) * p.row_group_stride : m0;
+    V.orow0 = (uint32_t)orow0;
+    V.res = make_rsrc((const bf16_t*)p.residual + orow0 * p.ldr,
+                      p.residual ? rec_bytes((out_row(p, p.m - 1) + 1 - orow0) * p.ldr * 2) : 0u);
     const int64_t pp = p.pos_period > 0 ? p.pos_period : 1;
     V.pos = make_rsrc(p.pos, p.pos ? rec_bytes(pp * p.ldp * 2) : 0u);
   }
@@ -241,7 +230,7 @@ __device__ __forceinline__ void epi_load_row(const GemmArgs& p, const EpiViews& 
                                              int64_t n, bool vec, int cnt, EpiIn& in) {
   if (MODE == FVX_GEMM_GEGLU) return;
   if constexpr (SP) {
-    const uint32_t ml = (uint32_t)m - (uint32_t)V.m0;
+    const uint32_t ml = (uint32_t)m - V.m0;
     in.res = bl_b8(V.res, (ml * (uint32_t)p.ldr + (uint32_t)n) * 2u, vec);
     in.gate = bl_b8(V.gate, (ml * (uint32_t)p.ldg + (uint32_t)n) * 2u, vec);
     return;
@@ -250,8 +239,8 @@ __device__ __forceinline__ void epi_load_row(const GemmArgs& p, const EpiViews& 
     const int hd = p.head_dim;
     const bool rot = n < (int64_t)(p.n_q_heads + 1) * hd;
     const int64_t pos =
-        (int32_t)__builtin_amdgcn_raw_buffer_load_b32(V.positions, (uint32_t)((m - V.m0) * 4),
-                                                      0, 0);
+        (int32_t)__builtin_amdgcn_raw_buffer_load_b32(V.positions, ((uint32_t)m - V.m0) * 4u, 0,
+                                                      0);
     bl_f8(V.rope, rot ? (uint32_t)((pos * (hd >> 1) + (umod32(n, hd) >> 1)) * 8) : kOOB, vec,
           in.f0);
     return;
@@ -263,19 +252,21 @@ __device__ __forceinline__ void epi_load_row(const GemmArgs& p, const EpiViews& 
   if (p.rtc_lock) in.locked = rr < *(const __attribute__((address_space(4))) int32_t*)p.rtc_lock;
   if (p.bias_f32_locked) {  // (f0 holds the unlocked rows' bias: epi_load_col)
     float fl[8];
-    bl_f8(V.bf32l, (uint32_t)(n * 4), vec, fl);
+    bl_f8(make_rsrc(p.bias_f32_locked, rec_bytes(p.n * 4)), (uint32_t)(n * 4), vec, fl);
 #pragma unroll
     for (int e = 0; e < 8; ++e) in.f0[e] = in.locked ? fl[e] : in.f0[e];
   }
   if (MODE == FVX_GEMM_EULER) {
-    bl_f8(V.xt, (uint32_t)(((m - V.m0) * p.ldx + n) * 4), vec, in.xt);
-    bl_f8(V.prev, (uint32_t)(((m - V.m0) * p.ld_prev + n) * 4), vec, in.prev);
+    const uint32_t ml = (uint32_t)m - V.m0;
+    bl_f8(V.xt, (ml * (uint32_t)p.ldx + (uint32_t)n) * 4u, vec, in.xt);
+    bl_f8(V.prev, (ml * (uint32_t)p.ld_prev + (uint32_t)n) * 4u, vec, in.prev);
     in.cw = bload1f(V.cw, (uint32_t)(rr * 4));
     return;
   }
-  const int64_t grow = (p.gate_group > 1 ? udiv32(m, p.gate_group) : m) - V.grow0;
-  in.gate = bl_b8(V.gate, (uint32_t)((grow * p.ldg + n) * 2), vec);
-  in.res = bl_b8(V.res, (uint32_t)(((out_row(p, m) - V.orow0) * p.ldr + n) * 2), vec);
+  const uint32_t grow = (p.gate_group > 1 ? udiv32(m, p.gate_group) : (uint32_t)m) - V.grow0;
+  in.gate = bl_b8(V.gate, (grow * (uint32_t)p.ldg + (uint32_t)n) * 2u, vec);
+  const uint32_t orow = (uint32_t)out_row(p, m) - V.orow0;
+  in.res = bl_b8(V.res, (orow * (uint32_t)p.ldr + (uint32_t)n) * 2u, vec);
   in.pos = bl_b8(V.pos,
                  (uint32_t)(((p.pos_period > 1 ? umod32(m, p.pos_period) : 0) * p.ldp + n) * 2),
                  vec);

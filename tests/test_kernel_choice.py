@@ -42,7 +42,7 @@ def test_row_major_head_dim_256(rows, problems, sk, splits):
 @pytest.mark.parametrize('rows,problems,tiles,splits', [
     (64, 1, 8, 1), (64, 1, 9, 5), (64, 31, 9, 5), (64, 32, 9, 1), (64, 32, 10, 5),
     (64, 1, 64, 32), (1, 1, 64, 32), (64, 4, 16, 8), (64, 16, 8, 1),
-    (256, 16, 4, 1), (64, 48, 11, 1), (64, 48, 14, 4), (64, 64, 20, 1), (64, 64, 32, 3),
+    (256, 16, 4, 1), (64, 48, 11, 1), (64, 48, 14, 1), (64, 48, 16, 4), (64, 64, 20, 1), (64, 64, 32, 3),
     (64, 80, 96, 1), (256, 64, 64, 1)])
 def test_unmasked_one_head(rows, problems, tiles, splits):
     assert _splits(_attn(rows, 64 * tiles, 72, problems=problems)) == splits
