@@ -1086,7 +1086,11 @@ __global__ __launch_bounds__(256, 1) void gemm_wide_f8_kernel(GemmArgs p, int m_
   const int64_t nn = n0 + wn * WNO + 8 * ch;
   const int cnt = (int)(N - nn < 8 ? N - nn : 8);
   const bool ho = (MODE == FVX_GEMM_PLAIN || GG) && (p.ss_out || p.a8_out);
-  const EpiViews V = epi_views<MODE>(p, m0);
+  // (the views' arithmetic stays behind the K loop: hoisted, its scalars spill and the
+  // K ranges of the prefix down lose 1 us of 75)
+  int me = (int)m0;
+  asm volatile("" : "+s"(me));
+  const EpiViews V = epi_views<MODE>(p, me);
   auto to_scr = [&](auto ic) {
     constexpr int i = decltype(ic)::value;
 #pragma unroll
