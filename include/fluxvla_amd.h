@@ -356,8 +356,9 @@ int fvx_adarms_norm_locked(const void* x, const void* style,
  * kgrp/qgrp means no mask.  This encodes make_att_2d_masks
  * (fluxvla/engines/utils/model_utils.py:77-95): kgrp = pad ? cumsum(att) :
  * INT32_MAX, qgrp = cumsum(att).  Rows that see no key produce zeros.
- * kv_splits > 1 splits the key range across workgroups (needs workspace; at
- * most 16384 ranges), 0 chooses, from the workspace that is there, 1 does not;
+ * kv_splits > 1 splits the key range across workgroups (needs workspace; the
+ * general kernel takes at most 16384 ranges), 0 chooses (the general kernel: as
+ * many as the workspace holds), 1 does not split;
  * the split partials are merged by a second kernel on the same stream, or,
  * for key ranges of fewer than 4 tiles (the bs=1 action expert) with
  * sq * heads % 8 == 0, by merging workgroups of the same launch: each
